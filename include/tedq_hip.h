@@ -50,6 +50,14 @@ int tedq_sv_build_tables(const void* params, int params_are_f64, int64_t batch, 
                          const void* slot_recs, int n_slots, const void* comp_recs, const void* const_pool,
                          void* mats, int64_t mat_stride, void* amats, int* err_flag, void* stream);
 
+/* The same for a lifted plan (tedq_amd/engine/lift.py): also fills the table
+ * parts of its rounds of reg_bits register bits.  round_recs: dev int32
+ * [n_rounds][18] (RoundRec in csrc/sv_tables.hip). */
+int tedq_sv_build_lift_tables(const void* params, int params_are_f64, int64_t batch, int n_params,
+                              const void* slot_recs, int n_slots, const void* comp_recs, const void* const_pool,
+                              void* mats, int64_t mat_stride, void* amats, int* err_flag, const void* round_recs,
+                              int n_rounds, int reg_bits, void* stream);
+
 /* ---- fused passes ---------------------------------------------------------- */
 /* One forward pass (a tile of 2^tile_bits amplitudes per workgroup, register
  * stages of 2^reg_bits amplitudes per thread) over every circuit; dev_prog is
@@ -87,6 +95,18 @@ int tedq_sv_adjoint_pass(void* psi, void* lam, int64_t batch, int n_qubits, int 
  * reference SV loop (pytorch_backend.py:358-380) and its autograd backward. */
 int tedq_sv_pass_ragged(int adjoint, const void* dev_recs, int n_recs, int64_t total_tiles, int k, int r,
                         void* stream);
+/* tedq_sv_apply_pass (flags bit 0 clear; lam, partials unused) or
+ * tedq_sv_adjoint_pass (bit 0 set; reg_bits <= 4) for a lifted plan's program
+ * (tedq_amd/engine/lift.py; stage words in csrc/sv_lift.hip), whose ops drop
+ * global phases.  flags bit 1: the pass has general ops. */
+int tedq_sv_lift_pass(int flags, void* psi, void* lam, int64_t batch, int n_qubits, int tile_bits, int reg_bits,
+                      int threads_log2, const int* dev_prog, uint64_t tile_mask, uint64_t zero_mask,
+                      const void* mats, int64_t mat_stride, float* partials, int64_t partial_rows, int n_gslots,
+                      void* stream);
+/* tedq_sv_pass_ragged for lifted programs; flags as tedq_sv_lift_pass (bit 1:
+ * some record's pass has general ops). */
+int tedq_sv_lift_pass_ragged(int flags, const void* dev_recs, int n_recs, int64_t total_tiles, int k, int r,
+                             void* stream);
 /* grad[b][p] = 2 Re sum_ij A[b][p][ij] C[b][g(p)][ij] with C reduced in fp64
  * (compensated) from the partial rows; grad is float32 or float64
  * (grad_is_f64).  pgslot: dev int32 [n_params]; C: dev double scratch

@@ -10,7 +10,9 @@
 namespace tedq {
 
 enum OpCode : int {
-  kOpU1 = 1, kOpD1 = 2, kOpCU1 = 3, kOpCX = 4, kOpCZ = 5,  // 6: unused
+  kOpU1 = 1, kOpD1 = 2, kOpCU1 = 3, kOpCX = 4, kOpCZ = 5,
+  // dense 4x4 at word[4] on bits word[1] > word[2] (the first the more significant index bit); lifted passes
+  kOpU2 = 6,
   kOpGrad1 = 7, kOpCGrad1 = 8, kOpCD1 = 9,
   // real 2x2 (imaginary parts of the table entries are zero), optionally controlled
   kOpR1 = 10,
@@ -23,6 +25,9 @@ enum OpCode : int {
   // amplitudes whose bit is 1 (and all control bits) times the slot's entry 1 (its conjugate with the
   // dagger flag): a diagonal gate without its global phase (the slot table stores p = d1 conj(d0) there)
   kOpPhase1 = 13,
+  // controlled phase of a lifted pass: amplitudes whose bit and control bits are all 1 times the complex
+  // number at word[4] (its conjugate with the dagger flag)
+  kOpPhaseLift = 15,
 };
 
 // kinds of kOpPauliGrad: the value equals 2 Re sum_ab A_ab C_ab for A = dU U^dagger of RX (X), RY (Y),
@@ -130,6 +135,129 @@ struct R1Op {  // real 2x2 on bit B where all CM bits are 1 (half the arithmetic
     }
   }
 };
+
+// ---------------------------------------------------------------------------
+// pieces of a lifted round (tedq_amd/engine/lift.py)
+// ---------------------------------------------------------------------------
+// The two numbers that RX (KIND 0) or RY (KIND 1) rotates into each other, for component c = 0, 1 of an amplitude
+// pair (x, y): RY (x, y) component by component, RX (y.im, x.re) and (x.im, y.re).
+template <int KIND>
+__device__ __forceinline__ float& rot_a(float2& x, float2& y, int c) {
+  return KIND == 1 ? (c ? x.y : x.x) : (c ? x.y : y.y);
+}
+template <int KIND>
+__device__ __forceinline__ float& rot_b(float2& x, float2& y, int c) {
+  return KIND == 1 ? (c ? y.y : y.x) : (c ? y.x : x.x);
+}
+
+// A rotation on bit B without its factor: (a, b) -> (a - q b, b + q a), with COT (q a - b, q b + a); DAG: the
+// transposed.
+template <int R, int B, int KIND, bool COT, bool DAG>
+__device__ __forceinline__ void rotate_unscaled(float2 (&v)[R], float q) {
+  const float s = DAG ? -1.f : 1.f;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i & (1 << B)) continue;
+    float2 &x = v[i], &y = v[i | (1 << B)];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      float &a = rot_a<KIND>(x, y, c), &b = rot_b<KIND>(x, y, c);
+      const float t = a;
+      a = COT ? fmaf(q, a, -s * b) : fmaf(-s * q, b, a);
+      b = COT ? fmaf(q, b, s * t) : fmaf(s * q, t, b);
+    }
+  }
+}
+struct Assign {
+  __device__ __forceinline__ void operator()(float& x, float t) const { x = t; }
+};
+
+template <int R>
+__device__ __forceinline__ void scale_all(float2 (&v)[R], float f) {
+#pragma unroll
+  for (int m = 0; m < R; ++m) {
+    v[m].x *= f;
+    v[m].y *= f;
+  }
+}
+
+// v_m *= d_m (DAG: conj d_m)
+template <int R, bool DAG, class SET>
+__device__ __forceinline__ void scale_diagonal(float2 (&v)[R], const float2* __restrict__ d, SET set) {
+#pragma unroll
+  for (int m = 0; m < R; ++m) {
+    const float2 c = d[m];
+    const float im = DAG ? -c.y : c.y;
+    const float t = fmaf(-v[m].y, im, v[m].x * c.x);
+    v[m].y = fmaf(v[m].x, im, v[m].y * c.x);
+    set(v[m].x, t);
+  }
+}
+
+template <int R>
+__device__ __forceinline__ void round_signs(float2 (&v)[R], uint32_t sign) {
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const uint32_t s = (sign << (31 - i)) & 0x80000000u;
+    v[i].x = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i].x) ^ s);
+    v[i].y = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i].y) ^ s);
+  }
+}
+
+// dense 4x4 (row-major, index bits (B1, B0), B1 > B0) on groups of four amplitudes
+template <int R, int B1, int B0>
+struct U2Op {
+  static __device__ __forceinline__ void run(float2 (&v)[R], const float2* __restrict__ m) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if (i & ((1 << B1) | (1 << B0))) continue;
+      const int j[4] = {i, i | (1 << B0), i | (1 << B1), i | (1 << B0) | (1 << B1)};
+      float2 o[4];
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        o[a] = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const float2 u = m[a * 4 + b], x = v[j[b]];
+          o[a].x = fmaf(u.x, x.x, fmaf(-u.y, x.y, o[a].x));
+          o[a].y = fmaf(u.x, x.y, fmaf(u.y, x.x, o[a].y));
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < 4; ++a) v[j[a]] = o[a];
+    }
+  }
+};
+
+constexpr int log2c(int x) { return x <= 1 ? 0 : 1 + log2c(x >> 1); }
+
+
+// Gradient values of the diagonal gates on all register bits at once: with w_m = Im conj(lambda_m) psi_m, bit b's RZ
+// value is the sum of w over bit b = 0 minus that over bit b = 1 (into acc[4 + b]); a PhaseShift's (bits of
+// kindp) is that minus the sum of all w.  The sums share their partial sums, one pairwise level per bit.
+template <int R>
+__device__ __forceinline__ void phase_grads(const float2 (&p)[R], const float2 (&l)[R], int bits, int kindp,
+                                            float (&acc)[8]) {
+  constexpr int r = log2c(R);
+  float w[R], g[r];
+#pragma unroll
+  for (int m = 0; m < R; ++m) w[m] = fmaf(l[m].x, p[m].y, -l[m].y * p[m].x);
+#pragma unroll
+  for (int b = 0; b < r; ++b) {
+    const int h = R >> (b + 1);
+    float d = 0.f;
+#pragma unroll
+    for (int m = 0; m < h; ++m) {
+      const float a = w[2 * m], c = w[2 * m + 1];
+      d += a - c;
+      w[m] = a + c;
+    }
+    g[b] = d;
+  }
+#pragma unroll
+  for (int b = 0; b < (r < 4 ? r : 4); ++b)
+    if ((bits >> b) & 1) acc[4 + b] += (kindp >> b) & 1 ? g[b] - w[0] : g[b];
+}
 
 // Gradient value of a one-parameter rotation (see PauliGradKind) over the pairs of bit B where all CM
 // bits are 1; NEG flips the sign (a daggered gate).  X: Im C01 + Im C10, Y: Re C10 - Re C01,

@@ -25,12 +25,21 @@ enum GateCode : int {
 
 // scalar: 0 for a slot whose gradients use the full bilinears C_ij of its gslot; c + 1 when the slot's
 // one trainable parameter gets its gradient value directly in component c of gslot (kOpPauliGrad): then
-// A is the constant that picks that component out of 2 Re sum A_ij C_ij.
+// A is the constant that picks that component out of 2 Re sum A_ij C_ij (negative: its negative).
 struct SlotRec {
   // phase = 1: a diagonal slot diag(d0, d1) also stores p = d1 conj(d0) in its (zero) entry 1, the phase
   // that kOpPhase1 applies to the |1> half (the gate up to its global phase d0)
-  int kind, ncomp, comp_start, mat_off, gslot, scalar, phase, pad2;
+  // form (kForm*, lifted plans): parts of a round have no row of their own (k_build_tables' second part)
+  int kind, ncomp, comp_start, mat_off, gslot, scalar, phase, form;
 };
+enum SlotForm : int { kFormX = 1, kFormY = 2, kFormDiag = 3, kFormEuler = 4, kFormPhase = 5, kFormDense = 6 };
+
+// A round of a lifted plan: table offset, whether it has a D0, and the slots (or -1) of D0, the rotations and
+// D1 on each register bit.
+struct RoundRec {
+  int coef, has_d0, pre[5], rot[5], post[5], pad;
+};
+static_assert(sizeof(RoundRec) == 72, "18 words (ROUND_WORDS of tedq_amd/engine/lift.py)");
 struct CompRec {
   int code, dagger, src0, src1, src2, const_off, pad0, pad1;
 };
@@ -161,11 +170,110 @@ __device__ M2 comp_eval(const CompRec& cr, const PT* prow, const double2* cpool,
   return cr.dagger ? m2_dag(m) : m;
 }
 
+__device__ __forceinline__ cd cd_unit(cd a) {
+  const double r = sqrt(a.x * a.x + a.y * a.y);
+  return r > 0.0 ? mkcd(a.x / r, a.y / r) : mkcd(1, 0);
+}
+
+template <typename PT>
+__device__ M2 slot_matrix(const SlotRec& sr, const CompRec* __restrict__ comps, const PT* prow,
+                          const double2* __restrict__ cpool, bool* ok) {
+  bool ok1;
+  M2 S = m2_eye();
+  *ok = true;
+  for (int c = 0; c < sr.ncomp; ++c) {
+    S = m2_mul(comp_eval(comps[sr.comp_start + c], prow, cpool, -1, &ok1), S);
+    *ok = *ok && ok1;
+  }
+  return S;
+}
+
+__device__ __forceinline__ double shfl_d(double v, int lane) { return __shfl(v, lane, 64); }
+
+// Table row part of one round, by 32 lanes: lanes 0..4 evaluate the D0 slot of their bit, 8..12 the rotation,
+// 16..20 the D1 slot, then lane m writes entry m of the diagonals.  A rotation [[c, -s], [s, c]] is stored as
+// q = s / c with factor c, or as q = c / s with factor s (the second form), |q| <= 1;
+// a general slot
+// S = e^id [[c, -s e^ig], [s e^ia, c e^i(a+g)]] is e^ig on bit 1, the rotation, e^ia on bit 1: a from S10 / S00
+// (any phase where one of them is 0), g from arg S11 / S00 = a + g or arg -S01 / S10 = g - a, whichever
+// entries are larger.
+template <typename PT>
+__device__ void round_row(const RoundRec& rr, int r, const SlotRec* __restrict__ slots,
+                          const CompRec* __restrict__ comps, const double2* __restrict__ cpool, const PT* prow,
+                          float2* out, int* err) {
+  const int lane = threadIdx.x & 63, sub = lane & 31, base = lane & 32;
+  const int b = sub & 7, part = sub >> 3;
+  int si = -1;
+  if (b < r && b < 5) si = part == 0 ? rr.pre[b] : part == 1 ? rr.rot[b] : part == 2 ? rr.post[b] : -1;
+  // pre / post: the phase of the |1> half; rotations: their factor and, for general slots, both phases
+  cd before = mkcd(1, 0), after = mkcd(1, 0);
+  double factor = 1.0;
+  int cot = 0;
+  if (si >= 0) {
+    const SlotRec sr = slots[si];
+    bool ok;
+    const M2 S = slot_matrix(sr, comps, prow, cpool, &ok);
+    if (!ok) atomicOr(err, 1);
+    if (part != 1) {
+      before = cd_mul(S.a[3], cd_conj(S.a[0]));
+    } else {
+      double c = S.a[0].x, s = sr.form == kFormX ? -S.a[2].y : S.a[2].x;
+      if (sr.form == kFormEuler) {
+        c = sqrt(S.a[0].x * S.a[0].x + S.a[0].y * S.a[0].y);
+        s = sqrt(S.a[2].x * S.a[2].x + S.a[2].y * S.a[2].y);
+        after = cd_unit(cd_mul(S.a[2], cd_conj(S.a[0])));
+        if (c >= s) {
+          before = cd_unit(cd_mul(cd_mul(S.a[3], cd_conj(S.a[0])), cd_conj(after)));
+        } else {
+          const cd q = cd_mul(S.a[1], cd_conj(S.a[2]));
+          before = cd_unit(cd_mul(mkcd(-q.x, -q.y), after));
+        }
+      }
+      cot = fabs(s) > fabs(c);
+      // the factor follows from q as it is stored: the matrix is then orthogonal up to the factor's rounding
+      const float q = (float)(cot ? c / s : s / c);
+      factor = copysign(1.0 / sqrt(1.0 + (double)q * q), cot ? s : c);
+      out[(1 << r) + b] = make_float2(q, 0.f);
+    }
+  }
+  const int m = sub;
+  cd d0 = mkcd(1, 0), d1 = mkcd(1, 0);
+  double f = 1.0;
+  int cots = 0;
+  for (int j = 0; j < r; ++j) {
+    const cd p = mkcd(shfl_d(before.x, base + j), shfl_d(before.y, base + j));
+    const cd eb = mkcd(shfl_d(before.x, base + 8 + j), shfl_d(before.y, base + 8 + j));
+    const cd ea = mkcd(shfl_d(after.x, base + 8 + j), shfl_d(after.y, base + 8 + j));
+    const cd q = mkcd(shfl_d(before.x, base + 16 + j), shfl_d(before.y, base + 16 + j));
+    f *= shfl_d(factor, base + 8 + j);
+    cots |= __shfl(cot, base + 8 + j, 64) << j;
+    if ((m >> j) & 1) {
+      d0 = cd_mul(d0, cd_mul(p, eb));
+      d1 = cd_mul(d1, cd_mul(ea, q));
+    }
+  }
+  const int R = 1 << r;
+  if (m < R) {
+    out[m] = make_float2((float)(f * d1.x), (float)(f * d1.y));
+    if (rr.has_d0) out[R + r + 1 + m] = make_float2((float)d0.x, (float)d0.y);
+  }
+  if (m == 0) out[R + r] = make_float2(__builtin_bit_cast(float, cots), 0.f);
+}
+
 template <typename PT>
 __global__ void k_build_tables(const PT* __restrict__ params, int64_t batch, int n_params,
                                const SlotRec* __restrict__ slots, int nslots, const CompRec* __restrict__ comps,
                                const double2* __restrict__ cpool, float2* __restrict__ mats, int64_t mat_stride,
-                               double2* __restrict__ amats, int* __restrict__ err) {
+                               double2* __restrict__ amats, int* __restrict__ err,
+                               const RoundRec* __restrict__ rounds, int nrounds, int r, unsigned slot_blocks) {
+  if (blockIdx.x >= slot_blocks) {  // rounds of a lifted plan, 32 lanes each
+    const int64_t i = (int64_t)(blockIdx.x - slot_blocks) * (blockDim.x >> 5) + (threadIdx.x >> 5);
+    if (i >= batch * nrounds) return;
+    const int64_t b = i / nrounds;
+    const RoundRec rr = rounds[i - b * nrounds];
+    round_row(rr, r, slots, comps, cpool, params + b * (int64_t)n_params, mats + b * mat_stride + rr.coef, err);
+    return;
+  }
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= batch * nslots) return;
   const int64_t b = gid / nslots;
@@ -179,25 +287,29 @@ __global__ void k_build_tables(const PT* __restrict__ params, int64_t batch, int
       for (int j = 0; j < 4; ++j) {
         double2 v = cr.dagger ? cpool[cr.const_off + j * 4 + i] : cpool[cr.const_off + i * 4 + j];
         out[i * 4 + j] = make_float2((float)v.x, (float)(cr.dagger ? -v.y : v.y));
+        // lifted plans: the adjoint matrix follows
+        if (sr.form) out[16 + j * 4 + i] = make_float2((float)v.x, (float)(cr.dagger ? v.y : -v.y));
       }
     return;
   }
   bool ok = true, ok1;
   M2 S = m2_eye();
-  for (int c = 0; c < sr.ncomp; ++c) {
-    S = m2_mul(comp_eval(comps[sr.comp_start + c], prow, cpool, -1, &ok1), S);
-    ok = ok && ok1;
+  // (a lifted plan's rounds evaluate the slots that are part of them)
+  if (sr.form == 0 || sr.form == kFormPhase) {
+    S = slot_matrix(sr, comps, prow, cpool, &ok);
+    for (int i = 0; i < 4; ++i) out[i] = make_float2((float)S.a[i].x, (float)S.a[i].y);
+    if (sr.form == kFormPhase) out[0] = out[3];
   }
-  for (int i = 0; i < 4; ++i) out[i] = make_float2((float)S.a[i].x, (float)S.a[i].y);
   if (sr.phase) {
     const cd p = cd_mul(S.a[3], cd_conj(S.a[0]));
     out[1] = make_float2((float)p.x, (float)p.y);
   }
   if (!ok) atomicOr(err, 1);
   if (amats == nullptr || sr.gslot < 0) return;
-  if (sr.scalar > 0) {
+  if (sr.scalar != 0) {
     // component c = Re (even) or Im (odd) of C_{c/2}: A_{c/2} = 1/2 or -i/2, the other entries 0
-    const int c = sr.scalar - 1;
+    const int c = (sr.scalar > 0 ? sr.scalar : -sr.scalar) - 1;
+    const double h = sr.scalar > 0 ? 0.5 : -0.5;
     for (int k = 0; k < sr.ncomp; ++k) {
       const CompRec cr = comps[sr.comp_start + k];
       const int srcs[3] = {cr.src0, cr.src1, cr.src2};
@@ -205,7 +317,7 @@ __global__ void k_build_tables(const PT* __restrict__ params, int64_t batch, int
         if (srcs[w] == INT32_MIN || srcs[w] < 0) continue;
         double2* dst = amats + (b * (int64_t)n_params + srcs[w]) * 4;
         for (int i = 0; i < 4; ++i)
-          dst[i] = i == (c >> 1) ? ((c & 1) ? make_double2(0.0, -0.5) : make_double2(0.5, 0.0))
+          dst[i] = i == (c >> 1) ? ((c & 1) ? make_double2(0.0, -h) : make_double2(h, 0.0))
                                  : make_double2(0.0, 0.0);
       }
     }
@@ -390,36 +502,57 @@ __global__ void k_tn_param_grad(const float2* __restrict__ env, int64_t env_stri
 
 using namespace tedq;
 
-extern "C" int tedq_sv_build_tables(const void* params, int params_are_f64, int64_t batch, int n_params,
-                                    const void* slot_recs, int n_slots, const void* comp_recs,
-                                    const void* const_pool, void* mats, int64_t mat_stride, void* amats,
-                                    int* err_flag, void* stream) {
-  if (batch <= 0 || n_slots < 0 || n_params < 0 || mats == nullptr || err_flag == nullptr) {
-    set_error("tedq_sv_build_tables: bad arguments (batch=%lld slots=%d params=%d)", (long long)batch, n_slots,
-              n_params);
+static int build_tables(const char* what, const void* params, int params_are_f64, int64_t batch, int n_params,
+                        const void* slot_recs, int n_slots, const void* comp_recs, const void* const_pool, void* mats,
+                        int64_t mat_stride, void* amats, int* err_flag, const void* round_recs, int n_rounds, int r,
+                        void* stream) {
+  if (batch <= 0 || n_slots < 0 || n_params < 0 || mats == nullptr || err_flag == nullptr || n_rounds < 0 ||
+      (n_rounds > 0 && (round_recs == nullptr || r < 1 || r > 5))) {
+    set_error("%s: bad arguments (batch=%lld slots=%d params=%d)", what, (long long)batch, n_slots, n_params);
     return kBadArgument;
   }
   if (n_slots == 0) return kOk;
   if (n_params > 0 && params == nullptr) {
-    set_error("tedq_sv_build_tables: params pointer is null");
+    set_error("%s: params pointer is null", what);
     return kBadArgument;
   }
-  const int64_t total = batch * n_slots;
   const int threads = 128;
-  const int64_t blocks = (total + threads - 1) / threads;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (params_are_f64) {
-    hipLaunchKernelGGL(k_build_tables<double>, dim3((unsigned)blocks), dim3(threads), 0, st,
-                       static_cast<const double*>(params), batch, n_params, static_cast<const SlotRec*>(slot_recs),
-                       n_slots, static_cast<const CompRec*>(comp_recs), static_cast<const double2*>(const_pool),
-                       static_cast<float2*>(mats), mat_stride, static_cast<double2*>(amats), err_flag);
-  } else {
-    hipLaunchKernelGGL(k_build_tables<float>, dim3((unsigned)blocks), dim3(threads), 0, st,
-                       static_cast<const float*>(params), batch, n_params, static_cast<const SlotRec*>(slot_recs),
-                       n_slots, static_cast<const CompRec*>(comp_recs), static_cast<const double2*>(const_pool),
-                       static_cast<float2*>(mats), mat_stride, static_cast<double2*>(amats), err_flag);
+  const int64_t slot_blocks = (batch * n_slots + threads - 1) / threads;
+  const int64_t blocks = slot_blocks + (batch * n_rounds * 32 + threads - 1) / threads;
+  if (blocks > 0x7fffffffll) {
+    set_error("%s: grid too large (%lld blocks)", what, (long long)blocks);
+    return kBadArgument;
   }
-  return check_launch("tedq_sv_build_tables");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+#define TEDQ_TABLES(PT)                                                                                              \
+  hipLaunchKernelGGL(k_build_tables<PT>, dim3((unsigned)blocks), dim3(threads), 0, st, static_cast<const PT*>(params), \
+                     batch, n_params, static_cast<const SlotRec*>(slot_recs), n_slots,                               \
+                     static_cast<const CompRec*>(comp_recs), static_cast<const double2*>(const_pool),                \
+                     static_cast<float2*>(mats), mat_stride, static_cast<double2*>(amats), err_flag,                 \
+                     static_cast<const RoundRec*>(round_recs), n_rounds, r, (unsigned)slot_blocks)
+  if (params_are_f64)
+    TEDQ_TABLES(double);
+  else
+    TEDQ_TABLES(float);
+#undef TEDQ_TABLES
+  return check_launch(what);
+}
+
+extern "C" int tedq_sv_build_tables(const void* params, int params_are_f64, int64_t batch, int n_params,
+                                    const void* slot_recs, int n_slots, const void* comp_recs,
+                                    const void* const_pool, void* mats, int64_t mat_stride, void* amats,
+                                    int* err_flag, void* stream) {
+  return build_tables("tedq_sv_build_tables", params, params_are_f64, batch, n_params, slot_recs, n_slots, comp_recs,
+                      const_pool, mats, mat_stride, amats, err_flag, nullptr, 0, 0, stream);
+}
+
+extern "C" int tedq_sv_build_lift_tables(const void* params, int params_are_f64, int64_t batch, int n_params,
+                                         const void* slot_recs, int n_slots, const void* comp_recs,
+                                         const void* const_pool, void* mats, int64_t mat_stride, void* amats,
+                                         int* err_flag, const void* round_recs, int n_rounds, int reg_bits,
+                                         void* stream) {
+  return build_tables("tedq_sv_build_lift_tables", params, params_are_f64, batch, n_params, slot_recs, n_slots,
+                      comp_recs, const_pool, mats, mat_stride, amats, err_flag, round_recs, n_rounds, reg_bits, stream);
 }
 
 extern "C" int tedq_tn_gate_tensors(const void* params, int params_are_f64, int64_t batch, int n_params,

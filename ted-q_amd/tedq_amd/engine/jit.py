@@ -20,9 +20,9 @@ import os
 
 import numpy as np
 
-from . import hip
+from . import hip, lift
 from .planner import (OP_U1, OP_D1, OP_CU1, OP_CX, OP_CZ, OP_GRAD1, OP_CGRAD1, OP_CD1, OP_R1, OP_PGRAD, OP_GFLUSH,
-                      OP_PH1)
+                      OP_PH1, OP_U2)
 from .program import HDR_TILE_BITS, HDR_HI_OFF, HDR_STAGES, STAGE_WORDS, OP_WORDS, lds_swizzle
 
 _CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))), "csrc")
@@ -155,6 +155,88 @@ def _op_lines(w, R, regs, adjoint, seg):
     return out
 
 
+def _group_lines(acc, gslot, seg):
+    """Write the 8 values ``acc`` to gradient slot ``gslot`` and clear them."""
+    return (["{", f"  float* dst = pbase + (int64_t){gslot} * a.np * 8;"] + _reduce_write_lines(acc, seg)
+            + ["#pragma unroll", f"  for (int q = 0; q < 8; ++q) {acc}[q] = 0.f;", "}"])
+
+
+def _round_lines(st, words, R, regs, adjoint, seg):
+    """Source lines of one round of a lifted program (lift.py) on the register arrays ``regs``."""
+    rots, grads, kindp = int(st[lift.W_ROT]), int(st[lift.W_GRADS]), int(st[lift.W_KINDP])
+    d1, sign, flags = int(st[lift.W_COEF]), int(st[lift.W_SIGN]) & 0xFFFFFFFF, int(st[lift.W_FLAGS])
+    out, r = [], R.bit_length() - 1
+    dagger = "true" if adjoint else "false"
+    rt, d0 = d1 + R, d1 + R + r + 1
+    cots = f"__builtin_bit_cast(int, mb[{rt + r}].x)"
+
+    def diagonal(flag, at):
+        if flags & flag:
+            out.extend(f"scale_diagonal<{R}, {dagger}>({v}, mb + {at}, Assign());" for v in regs)
+
+    def rotations(mask, kind):
+        for b in _bits(mask & 31):
+            for cot, cond in (("true", f"if (({cots} >> {b}) & 1)"), ("false", "else")):
+                runs = " ".join(f"rotate_unscaled<{R}, {b}, {kind}, {cot}, {dagger}>({v}, mb[{rt + b}].x);"
+                                for v in regs)
+                out.append(f"{cond} {{ {runs} }}")
+
+    def factor():
+        if flags & lift.HAS_SCALE:
+            out.extend(f"scale_all<{R}>({v}, mb[{d1}].x);" for v in regs)
+
+    def signs():
+        if sign:
+            out.extend(f"round_signs<{R}>({v}, {sign}u);" for v in regs)
+
+    def general():
+        for o in range(int(st[lift.W_NGEN])):
+            at = int(st[lift.W_GEN]) + o * OP_WORDS
+            w = words[at:at + OP_WORDS]
+            t, dag = int(w[0]) & 0xFF, (int(w[0]) >> 8) & 1
+            b, cm, off = int(w[1]), int(w[3]), int(w[4])
+            if t == OP_PGRAD:
+                kind, neg = int(w[6]) & 15, int(w[6]) >> 4
+                out.append("{ float gv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};")
+                out.append(f"PauliGradOp<{R}, {b}, {cm}, {kind}, {'true' if neg else 'false'}>::run(vp, vl, gv[0]);")
+                out.extend(_group_lines("gv", int(w[5]), seg) + ["}"])
+            elif t == OP_U2:
+                out.extend(f"U2Op<{R}, {b}, {int(w[2])}>::run({v}, mb + {off});" for v in regs)
+            elif t == lift.OP_PHL:
+                p = f"cconj(mb[{off}])" if dag else f"mb[{off}]"
+                out.extend(f"DiagOp<{R}, {b}, {cm | (1 << b)}>::run({v}, {p}, {p});" for v in regs)
+            else:
+                out.extend(_op_lines(w, R, regs, adjoint, seg))
+
+    if not adjoint:
+        diagonal(lift.HAS_D0, d0)
+        rotations(rots, 0)
+        rotations(rots >> 8, 1)
+        diagonal(lift.HAS_D1, d1)
+        factor()
+        general()
+        signs()
+        return out
+    signs()
+    general()
+    if (grads >> 8) & 31:
+        out.append(f"phase_grads<{R}>(vp, vl, {(grads >> 8) & 31}, {kindp & 31}, sacc);")
+    diagonal(lift.HAS_D1, d1)
+    factor()
+    rotations(rots, 0)
+    rotations(rots >> 8, 1)
+    for kind, sh in ((0, 0), (1, 8)):
+        for b in _bits(grads & (rots >> sh) & 31):
+            out.append(f"PauliGradOp<{R}, {b}, 0, {kind}, false>::run(vp, vl, sacc[{b}]);")
+    if int(st[lift.W_GROUP]) >= 0:
+        out.extend(_group_lines("sacc", int(st[lift.W_GROUP]), seg))
+    if int(st[lift.W_GROUP_PRE]) >= 0:
+        out.append(f"phase_grads<{R}>(vp, vl, {(grads >> 16) & 31}, {(kindp >> 8) & 31}, sacc);")
+        out.extend(_group_lines("sacc", int(st[lift.W_GROUP_PRE]), seg))
+    diagonal(lift.HAS_D0, d0)
+    return out
+
+
 def _seed_lines(hi, R, masks):
     """Per-register lambda / psi factors d_m = sum_j c_j (-1)^popc(x & mask_j) for x = rest bits | lane
     bits | register m's bits: the rest and lane parities per thread, the register parities as constants."""
@@ -174,7 +256,7 @@ def _seed_lines(hi, R, masks):
     return out
 
 
-def pass_kernel_source(name, words, adjoint, seed_masks=None, fresh=0, persistent=False):
+def pass_kernel_source(name, words, adjoint, seed_masks=None, fresh=0, persistent=False, lifted=False):
     """HIP source of one generated pass kernel from its program words (program.py layout).
 
     ``seed_masks`` (adjoint only): instead of loading lambda, form it from the loaded psi as
@@ -186,7 +268,8 @@ def pass_kernel_source(name, words, adjoint, seed_masks=None, fresh=0, persisten
     ``persistent`` (adjoint only; launched with kPassPersistent): each workgroup loops over the tiles
     blockIdx.x, blockIdx.x + gridDim.x, ... and loads the next tile's psi and lambda into registers
     while the current one is processed, so the load of a tile overlaps the arithmetic of the previous
-    one even where a single workgroup fills a CU's LDS."""
+    one even where a single workgroup fills a CU's LDS.
+    ``lifted``: the words are a lifted plan's (rounds, lift.py)."""
     words = np.asarray(words, dtype=np.int32)
     k, r, nst, tT = (int(x) for x in words[:4])
     R, T = 1 << r, 1 << tT
@@ -273,27 +356,39 @@ def pass_kernel_source(name, words, adjoint, seed_masks=None, fresh=0, persisten
         L += prefetch("TILE + gridDim.x", "lo")
     regs = ("vp", "vl") if adjoint else ("v",)
     for s in range(nst):
-        base = HDR_STAGES + STAGE_WORDS * s
-        nops, op_off, nonreg = int(words[base]), int(words[base + 1]), int(words[base + 2])
-        offs = [int(x) for x in words[base + 4:base + 4 + R]]
-        L.append("  {")
-        # the thread index is re-read through an empty asm in every stage: otherwise the compiler computes
-        # the LDS offsets of all stages up front and keeps them live (up to ~100 more VGPRs in long passes)
-        L.append('    int ts = threadIdx.x; asm volatile("" : "+v"(ts));')
-        L.append(f"    const int sb = swz({_pdep_expr('ts', _bits(nonreg))});")
-        for v in regs:
-            L.append(f"    float2 {v}[{R}];")
-        for m in range(R):
-            for v, arr in zip(regs, ("lds", "ldl")):
-                L.append(f"    {v}[{m}] = {arr}[sb ^ {offs[m]}];")
-        for o in range(nops):
-            w = words[op_off + o * OP_WORDS: op_off + (o + 1) * OP_WORDS]
-            L.extend("    " + x for x in _op_lines(w, R, regs, adjoint, seg))
-        for m in range(R):
-            for v, arr in zip(regs, ("lds", "ldl")):
-                L.append(f"    {arr}[sb ^ {offs[m]}] = {v}[{m}];")
-        L.append("    __syncthreads();")
-        L.append("  }")
+        sw_words = lift.STAGE_WORDS if lifted else STAGE_WORDS
+        st = words[HDR_STAGES + sw_words * s:HDR_STAGES + sw_words * (s + 1)]
+        if lifted:
+            flags, nonreg = int(st[lift.W_FLAGS]), ((1 << k) - 1) & ~int(st[lift.W_REGMASK])
+            offs = [int(x) for x in st[lift.W_IN:lift.W_IN + R]]
+            outs = [int(x) for x in st[lift.W_OUT:lift.W_OUT + R]]
+        else:
+            nops, op_off, nonreg, flags = int(st[0]), int(st[1]), int(st[2]), lift.BARRIER
+            offs = outs = [int(x) for x in st[4:4 + R]]
+        if not flags & lift.SKIP_READ:
+            L.append("  {")
+            # the thread index is re-read through an empty asm in every stage: otherwise the compiler computes
+            # the LDS offsets of all stages up front and keeps them live (up to ~100 more VGPRs in long passes)
+            L.append('    int ts = threadIdx.x; asm volatile("" : "+v"(ts));')
+            L.append(f"    const int sb = swz({_pdep_expr('ts', _bits(nonreg))});")
+            for v in regs:
+                L.append(f"    float2 {v}[{R}];")
+            for m in range(R):
+                for v, arr in zip(regs, ("lds", "ldl")):
+                    L.append(f"    {v}[{m}] = {arr}[sb ^ {offs[m]}];")
+        if lifted:
+            L.extend("    " + x for x in _round_lines(st, words, R, regs, adjoint, seg))
+        else:
+            for o in range(nops):
+                w = words[op_off + o * OP_WORDS: op_off + (o + 1) * OP_WORDS]
+                L.extend("    " + x for x in _op_lines(w, R, regs, adjoint, seg))
+        if not flags & lift.SKIP_WRITE:
+            for m in range(R):
+                for v, arr in zip(regs, ("lds", "ldl")):
+                    L.append(f"    {arr}[sb ^ {outs[m]}] = {v}[{m}];")
+            if flags & lift.BARRIER:
+                L.append("    __syncthreads();")
+            L.append("  }")
     if adjoint:
         # kPassPsiReadOnly: psi is a checkpoint of the forward; the state at this pass's start is the
         # previous checkpoint, so psi is not written back
@@ -329,15 +424,17 @@ def program_source(enc, n_fwd, n_adj, seed_masks=None, persistent=False, only=No
     for i in range(n_fwd):
         o = enc.fwd_offsets[i]
         if only is None or f"f{i}" in only:
-            parts.append(pass_kernel_source(f"f{i}", enc.prog[o:ends[o]], False, fresh=enc.tile_masks[i] & ~seen))
+            parts.append(pass_kernel_source(f"f{i}", enc.prog[o:ends[o]], False, fresh=enc.tile_masks[i] & ~seen,
+                                            lifted=enc.lift))
         seen |= enc.tile_masks[i]
     for i in range(n_adj):
         o = enc.adj_offsets[i]
         if only is None or f"a{i}" in only:
-            parts.append(pass_kernel_source(f"a{i}", enc.prog[o:ends[o]], True, persistent=persistent))
+            parts.append(pass_kernel_source(f"a{i}", enc.prog[o:ends[o]], True, persistent=persistent, lifted=enc.lift))
     if seed_masks is not None and n_adj and (only is None or "a0s" in only):
         o = enc.adj_offsets[0]
-        parts.append(pass_kernel_source("a0s", enc.prog[o:ends[o]], True, seed_masks, persistent=persistent))
+        parts.append(pass_kernel_source("a0s", enc.prog[o:ends[o]], True, seed_masks, persistent=persistent,
+                                        lifted=enc.lift))
     return "\n\n".join(parts) + "\n"
 
 

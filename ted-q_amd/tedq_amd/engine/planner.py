@@ -62,6 +62,8 @@ class Slot:
     mat_off: int = 0       # complex64 offset inside one batch row of the table
     gslot: int = -1        # gradient slot index or -1
     scomp: int = -1        # component inside gslot of a single-value gradient (OP_PGRAD), else -1
+    controlled: bool = False
+    form: int = 0          # lifted plans: how the table kernel stores it (lift.py)
 
     @property
     def dim(self):
@@ -94,10 +96,11 @@ class Slot:
 @dataclass
 class Unit:
     """A gate as the kernels see it: physical bits it touches and how to apply it."""
-    kind: str              # "u1", "cu1", "cx", "cz"
+    kind: str              # "u1", "cu1", "cx", "cz"; lifted plans also "u2" (bits: high, low)
     bits: tuple            # for u1/cu1/cx: (target, *controls); cz: all bits
     comp: Component = None
     index: int = 0
+    group: tuple = None    # units of one two-qubit user matrix: (constant offset of the 4x4, member number)
 
 
 @dataclass
@@ -124,6 +127,11 @@ class Plan:
     n_gslots: int
     mat_stride: int        # complex64 entries per batch row of the slot table
     specialize: bool = False   # adjoint plan of generated kernels (see build_plan)
+    rounds: list = None        # lifted plan of the interpreted kernels: rounds per pass (lift.py)
+
+    @property
+    def lift(self):
+        return self.rounds is not None
 
 
 def gate_to_units(n, gate, srcs, const_pool):
@@ -193,6 +201,10 @@ def two_qubit_units(m, b_hi, b_lo, const_pool):
     r1 = np.array([[cs[1, 1], cs[1, 3]], [cs[3, 1], cs[3, 3]]])
     units += _multiplexor(b_hi, b_lo, r0, r1, const_pool)
     units += _multiplexor(b_lo, b_hi, u[:2, :2], u[2:, 2:], const_pool)
+    off = len(const_pool)
+    const_pool.extend(np.asarray(m, dtype=np.complex128).reshape(-1).tolist())
+    for i, x in enumerate(units):
+        x.group = (off, i)
     return units
 
 
@@ -251,7 +263,7 @@ def compact_register(units, zmasks, n):
     if len(used) == n:
         return units, list(zmasks), n
     new = {b: i for i, b in enumerate(used)}
-    out = [Unit(u.kind, tuple(new[b] for b in u.bits), u.comp, u.index) for u in units]
+    out = [Unit(u.kind, tuple(new[b] for b in u.bits), u.comp, u.index, u.group) for u in units]
     masks = []
     for m in zmasks:
         masks.append(sum(1 << new[b] for b in used if (m >> b) & 1))
@@ -299,7 +311,7 @@ def _schedule(units, order, max_bits, seed_bits, allowed_bits=None):
     return done, chosen
 
 
-def build_plan(n, units, n_params, const_pool, k_max=12, r=4, coalesce_bits=3, specialize=False):
+def build_plan(n, units, n_params, const_pool, k_max=12, r=4, coalesce_bits=3, specialize=False, lift=False):
     """Partition ``units`` (program order) into passes and register stages.
 
     With ``specialize`` (the adjoint's plan) a trainable single-qubit gate is never fused with another
@@ -307,7 +319,14 @@ def build_plan(n, units, n_params, const_pool, k_max=12, r=4, coalesce_bits=3, s
     of RX / RY / RZ / PhaseShift (and controlled forms) is one value per parameter (OP_PGRAD, 2-4
     multiply-adds per amplitude pair) instead of the slot's 8 bilinears (16 per pair), collected in
     groups of 8 per register stage.  Its uncontrolled diagonal gates run as phases on the |1> half
-    (OP_PH1, one complex multiply per pair instead of two; see program.py)."""
+    (OP_PH1, one complex multiply per pair instead of two; see program.py).
+
+    ``lift`` (the interpreted kernels' specialised plan; implies ``specialize``): the ops of every stage are
+    grouped into rounds that update amplitudes in place (lift.py); "fwd": for forward sweeps only."""
+    if lift:
+        from .lift import lift_units  # pylint: disable=import-outside-toplevel
+        specialize = True
+        units = lift_units(units, const_pool)
     k = min(n, k_max)
     widest = max((len(u.bits) for u in units), default=1)
     if widest > k:
@@ -333,6 +352,11 @@ def build_plan(n, units, n_params, const_pool, k_max=12, r=4, coalesce_bits=3, s
         done_set = set(done)
         todo = [u for u in todo if u not in done_set]
         passes.append(_build_pass(units, done, tile_bits, r, slots, specialize))
+    if lift:
+        from .lift import assign_rounds  # pylint: disable=import-outside-toplevel
+        rounds, mat_off, gslot = assign_rounds(passes, slots, r, lift == "fwd")
+        return Plan(n=n, k=k, r=r, passes=passes, slots=slots, const_pool=np.asarray(const_pool, dtype=np.complex128),
+                    n_params=n_params, n_gslots=gslot, mat_stride=max(mat_off, 1), specialize=True, rounds=rounds)
     mat_off = 0
     for s in slots:
         s.mat_off = mat_off
@@ -398,8 +422,11 @@ def _build_pass(units, pass_units, tile_bits, r, slots, specialize=False):
                 stage.ops.append(("u1", reg_of[b], 0, 0, len(slots) - 1))
             elif u.kind == "cu1":
                 cmask = sum(1 << reg_of[c] for c in u.bits[1:])
-                slots.append(Slot(SLOT_1Q, [u.comp]))
+                slots.append(Slot(SLOT_1Q, [u.comp], controlled=True))
                 stage.ops.append(("cu1", reg_of[u.bits[0]], 0, cmask, len(slots) - 1))
+            elif u.kind == "u2":
+                slots.append(Slot(SLOT_2Q, [u.comp]))
+                stage.ops.append(("u2", reg_of[u.bits[0]], reg_of[u.bits[1]], 0, len(slots) - 1))
             elif u.kind == "cx":
                 cmask = sum(1 << reg_of[c] for c in u.bits[1:])
                 stage.ops.append(("cx", reg_of[u.bits[0]], 0, cmask, -1))

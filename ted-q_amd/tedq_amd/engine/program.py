@@ -9,6 +9,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
+from . import lift
 from .planner import (OP_U1, OP_D1, OP_CU1, OP_CX, OP_CZ, OP_GRAD1, OP_CGRAD1, OP_CD1, OP_R1, OP_PGRAD,
                       OP_GFLUSH, OP_PH1, OP_DAGGER, SLOT_1Q)
 
@@ -31,6 +32,8 @@ class EncodedPlan:
     comp_recs: np.ndarray     # int32 [ncomps, 8]
     const_pool: np.ndarray    # float64 [npool, 2]
     pgslot: np.ndarray        # int32 [n_params]: gradient slot of each trainable parameter
+    lift: bool = False        # rounds of lift.py (tedq_sv_lift_pass) instead of op lists
+    round_recs: np.ndarray = None   # lifted: int32 [rounds, lift.ROUND_WORDS] for the table kernel
 
 
 def lds_swizzle(e):
@@ -101,10 +104,9 @@ def _adj_op_words(op, slots, specialize=False):
     return words
 
 
-def _encode_pass(p, k, r, slots, adjoint, specialize=False):
-    nst = len(p.stages)
-    stages = list(reversed(p.stages)) if adjoint else p.stages
-    header = np.zeros(HDR_STAGES + STAGE_WORDS * nst, dtype=np.int64)
+def _header(p, k, r, nst, stage_words):
+    """Pass header words with room for the stages, and the physical offsets of its load layout."""
+    header = np.zeros(HDR_STAGES + stage_words * nst, dtype=np.int64)
     tT = k - r
     header[0], header[1], header[2], header[3] = k, r, nst, tT
     for i, b in enumerate(p.tile_bits):
@@ -112,6 +114,33 @@ def _encode_pass(p, k, r, slots, adjoint, specialize=False):
     hi = np.zeros(32, dtype=np.int64)
     for m in range(1 << r):
         hi[m] = _pdep(m << tT, p.tile_bits)
+    return header, hi
+
+
+def _encode_lifted(p, rounds, plan, adjoint):
+    """A pass of a lifted plan: the same header, lift.STAGE_WORDS words per round, then the general ops."""
+    stages, gens = lift.encode_rounds(rounds, plan, adjoint, _pdep, lds_swizzle)
+    header, hi = _header(p, plan.k, plan.r, len(stages), lift.STAGE_WORDS)
+    for i, w in enumerate(stages):
+        w[lift.W_GEN] = len(header) + w[lift.W_GEN] * OP_WORDS
+        header[HDR_STAGES + lift.STAGE_WORDS * i:HDR_STAGES + lift.STAGE_WORDS * (i + 1)] = w
+    return _finish(header, hi, gens)
+
+
+def _finish(header, hi, op_words):
+    words = (header & 0xFFFFFFFF).astype(np.uint32).view(np.int32).copy()
+    words[HDR_HI_OFF:HDR_HI_OFF + 64] = hi.view(np.int32)
+    body = np.asarray(op_words, dtype=np.int32).reshape(-1) if op_words else np.zeros(0, np.int32)
+    out = np.concatenate([words, body])
+    if len(out) % 2:
+        out = np.concatenate([out, np.zeros(1, np.int32)])
+    return out
+
+
+def _encode_pass(p, k, r, slots, adjoint, specialize=False):
+    nst = len(p.stages)
+    stages = list(reversed(p.stages)) if adjoint else p.stages
+    header, hi = _header(p, k, r, nst, STAGE_WORDS)
     op_words = []
     op_start = len(header)
     for s_idx, st in enumerate(stages):
@@ -139,27 +168,25 @@ def _encode_pass(p, k, r, slots, adjoint, specialize=False):
         for m in range(1 << r):
             header[base + 4 + m] = lds_swizzle(_pdep(m, st.reg_bits))
         op_words.extend(ops)
-    words = header.astype(np.int32)
-    words[HDR_HI_OFF:HDR_HI_OFF + 64] = hi.view(np.int32)
-    body = np.asarray(op_words, dtype=np.int32).reshape(-1) if op_words else np.zeros(0, np.int32)
-    out = np.concatenate([words, body])
-    if len(out) % 2:
-        out = np.concatenate([out, np.zeros(1, np.int32)])
-    return out
+    return _finish(header, hi, op_words)
 
 
 def encode_plan(plan):
     """Serialise forward and adjoint pass programs plus the slot tables."""
     chunks, fwd_off, adj_off, masks = [], [], [], []
     pos = 0
-    for p in plan.passes:
-        w = _encode_pass(p, plan.k, plan.r, plan.slots, adjoint=False, specialize=plan.specialize)
+    def encode(i, adjoint):
+        if plan.lift:
+            return _encode_lifted(plan.passes[i], plan.rounds[i], plan, adjoint)
+        return _encode_pass(plan.passes[i], plan.k, plan.r, plan.slots, adjoint, specialize=plan.specialize)
+    for i, p in enumerate(plan.passes):
+        w = encode(i, False)
         fwd_off.append(pos)
         chunks.append(w)
         pos += len(w)
         masks.append(sum(1 << b for b in p.tile_bits))
-    for p in reversed(plan.passes):
-        w = _encode_pass(p, plan.k, plan.r, plan.slots, adjoint=True, specialize=plan.specialize)
+    for i in reversed(range(len(plan.passes))):
+        w = encode(i, True)
         adj_off.append(pos)
         chunks.append(w)
         pos += len(w)
@@ -169,8 +196,11 @@ def encode_plan(plan):
     comp_list = []
     pgslot = np.full(max(plan.n_params, 1), -1, dtype=np.int32)
     for si, s in enumerate(plan.slots):
-        slot_recs[si] = [s.kind, len(s.comps), len(comp_list), s.mat_off, s.gslot, s.scomp + 1,
-                         int(_phase_slot(s, plan.specialize)), 0]
+        scalar = s.scomp + 1
+        if plan.lift and s.scomp >= 0 and s.form and not s.controlled and s.pauli[1]:
+            scalar = -scalar          # a daggered rotation of a round: the kernel sums its value unsigned
+        slot_recs[si] = [s.kind, len(s.comps), len(comp_list), s.mat_off, s.gslot, scalar,
+                         int(not plan.lift and _phase_slot(s, plan.specialize)), s.form if plan.lift else 0]
         for c in s.comps:
             srcs = list(c.srcs) + [NO_SRC] * (3 - len(c.srcs))
             comp_list.append([c.code, int(c.dagger), srcs[0], srcs[1], srcs[2], c.const_mat, 0, 0])
@@ -183,4 +213,5 @@ def encode_plan(plan):
     const_pool = np.stack([pool.real, pool.imag], axis=1).astype(np.float64)
     return EncodedPlan(prog=prog.astype(np.int32), fwd_offsets=fwd_off, adj_offsets=adj_off,
                        tile_masks=masks, slot_recs=slot_recs, comp_recs=comp_recs,
-                       const_pool=np.ascontiguousarray(const_pool), pgslot=pgslot)
+                       const_pool=np.ascontiguousarray(const_pool), pgslot=pgslot, lift=plan.lift,
+                       round_recs=lift.round_records(plan) if plan.lift else None)

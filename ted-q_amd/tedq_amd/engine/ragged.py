@@ -36,8 +36,8 @@ def shape_key(ex):
 
 
 def _records(items, adjoint):
-    """Record table of every pass index: (records array, [(start, count, tiles) per pass index])."""
-    per_pass = []
+    """Record table of every pass index: (records array, [(start, count, tiles, general ops) per pass index])."""
+    per_pass, general = [], []
     for it in items:
         prog = it["ex"].bwd if adjoint else it["ex"].fwd
         enc, plan = prog.enc, prog.plan
@@ -55,6 +55,9 @@ def _records(items, adjoint):
         for i, (off, mask) in enumerate(zip(offs, masks)):
             while len(per_pass) <= i:
                 per_pass.append([])
+                general.append(0)
+            if prog.general:
+                general[i] |= prog.general[len(offs) - 1 - i if adjoint else i]
             for b in range(B):
                 per_pass[i].append((it["psi"].data_ptr() + b * amp,
                                     it["lam"].data_ptr() + b * amp if adjoint else 0,
@@ -62,27 +65,42 @@ def _records(items, adjoint):
                                     it["partials"].data_ptr() + b * prow_bytes if adjoint else 0,
                                     full & ~mask, 1 << (n - plan.k), n, G if adjoint else 0))
     rows, bounds = [], []
-    for recs in per_pass:
+    for recs, gen in zip(per_pass, general):
         start = len(rows)
         end = 0
         for psi, lam, prg, mats, part, rest, tiles, n, g in recs:
             end += tiles
             rows.append((psi, lam, prg, mats, part, rest, end, n, g))
-        bounds.append((start, len(recs), end))
+        bounds.append((start, len(recs), end, gen))
     arr = np.array(rows, dtype=RECORD)
     return arr, bounds
 
 
-def _launch(arr, bounds, adjoint, k, r, dev, st):
+def _launch_all(its, adjoint, k, r, dev, st):
+    """Every pass of the items: lifted plans run on their own kernels (tedq_sv_lift_pass_ragged), so they and
+    plain plans (forward sweeps whose global phase shows) are launched apart.  Returns buffers to keep alive."""
+    keep = []
+    for lift in (True, False):
+        mine = [it for it in its if (it["ex"].bwd if adjoint else it["ex"].fwd).plan.lift == lift]
+        if mine:
+            arr, bounds = _records(mine, adjoint)
+            keep += _launch(arr, bounds, adjoint, lift, k, r, dev, st)
+    return keep
+
+
+def _launch(arr, bounds, adjoint, lift, k, r, dev, st):
     """Copy the record table to the device and issue one ragged launch per pass index."""
     host = torch.from_numpy(arr.view(np.uint8).copy()).pin_memory()
     table = torch.empty(host.shape, dtype=torch.uint8, device=dev)
     table.copy_(host, non_blocking=True)
-    for start, count, tiles in bounds:
+    for start, count, tiles, gen in bounds:
         if not count:
             continue
-        hip.call("tedq_sv_pass_ragged", int(adjoint), ctypes.c_void_p(table.data_ptr() + 64 * start), count, tiles,
-                 k, r, st)
+        recs = ctypes.c_void_p(table.data_ptr() + 64 * start)
+        if lift:
+            hip.call("tedq_sv_lift_pass_ragged", int(adjoint) + 2 * gen, recs, count, tiles, k, r, st)
+        else:
+            hip.call("tedq_sv_pass_ragged", int(adjoint), recs, count, tiles, k, r, st)
     return host, table
 
 
@@ -113,9 +131,7 @@ def ragged_value_and_grad(items, device):
         else:
             hip.call("tedq_sv_init_copy", hip.ptr(psi), hip.ptr(init), rows.shape[0], ex.n, st)
         its.append({"ex": ex, "rows": rows, "ups": ups, "dev": device, "mats_f": mats_f, "psi": psi})
-    keep = []
-    arr, bounds = _records(its, adjoint=False)
-    keep += _launch(arr, bounds, False, kf, rf, device, st)
+    keep = _launch_all(its, False, kf, rf, device, st)
     for it in its:
         ex = it["ex"]
         it["outs"] = ex.measure(it["psi"])
@@ -124,8 +140,7 @@ def ragged_value_and_grad(items, device):
         G = ex.bwd.plan.n_gslots
         it["partials"] = torch.empty((it["rows"].shape[0], max(G, 1), ex.bwd.partial_rows(), 8),
                                      dtype=torch.float32, device=device)
-    arr, bounds = _records(its, adjoint=True)
-    keep += _launch(arr, bounds, True, kb, rb, device, st)
+    keep += _launch_all(its, True, kb, rb, device, st)
     results = []
     for it in its:
         ex, rows = it["ex"], it["rows"]

@@ -127,6 +127,7 @@ class _DeviceBuffers:
         self.comp_recs = torch.from_numpy(enc.comp_recs.reshape(-1)).to(device)
         self.const_pool = torch.from_numpy(enc.const_pool.reshape(-1)).to(device)
         self.pgslot = torch.from_numpy(enc.pgslot).to(device)
+        self.round_recs = torch.from_numpy(enc.round_recs.reshape(-1)).to(device) if enc.lift else None
         self.prog_base = self.prog.data_ptr()
         # unknown-gate-code flag of the table builder (set once; never cleared inside a graph), read back
         # after the first table build that is not being captured into a graph
@@ -141,11 +142,13 @@ class _DeviceBuffers:
 class _Program:
     """One fusion plan (tile bits k, register bits r) with its encoded device program."""
 
-    def __init__(self, n, units, n_params, const_pool, k, r, specialize=False):
+    def __init__(self, n, units, n_params, const_pool, k, r, specialize=False, lift=False):
         self.n = n
         self.n_params = n_params
-        self.plan = build_plan(n, units, n_params, const_pool, k_max=k, r=r, specialize=specialize)
+        self.plan = build_plan(n, units, n_params, const_pool, k_max=k, r=r, specialize=specialize, lift=lift)
         self.enc = encode_plan(self.plan)
+        # lifted plans: whether a pass has general ops (1 or 0 per pass)
+        self.general = [int(any(rd.gen for rd in rounds)) for rounds in self.plan.rounds or []]
         self._dev = {}
         self._jit = {}          # device key -> JitModule of generated pass kernels
         # From |0..0>, before pass p the state vanishes wherever a bit that no earlier pass held in its tile
@@ -250,10 +253,14 @@ class _Program:
         # columns are never read (their gradient slot is -1)
         amats = torch.empty((B, max(self.n_params, 1), 4, 2), dtype=torch.float64, device=dev) if need_grad else None
         params = params.contiguous()
-        hip.call("tedq_sv_build_tables", hip.ptr(params) if self.n_params else None,
-                 int(params.dtype == torch.float64), B, self.n_params, hip.ptr(buf.slot_recs),
-                 len(self.plan.slots), hip.ptr(buf.comp_recs), hip.ptr(buf.const_pool), hip.ptr(mats),
-                 self.plan.mat_stride, hip.ptr(amats), hip.ptr(buf.err), hip.stream_handle(dev))
+        args = (hip.ptr(params) if self.n_params else None, int(params.dtype == torch.float64), B, self.n_params,
+                hip.ptr(buf.slot_recs), len(self.plan.slots), hip.ptr(buf.comp_recs), hip.ptr(buf.const_pool),
+                hip.ptr(mats), self.plan.mat_stride, hip.ptr(amats), hip.ptr(buf.err))
+        if self.plan.lift:
+            hip.call("tedq_sv_build_lift_tables", *args, hip.ptr(buf.round_recs), len(self.enc.round_recs), self.plan.r,
+                     hip.stream_handle(dev))
+        else:
+            hip.call("tedq_sv_build_tables", *args, hip.stream_handle(dev))
         if not buf.err_checked and not torch.cuda.is_current_stream_capturing():
             check_device_flag(buf.err, "tedq_sv_build_tables: a slot record holds an unknown gate code")
             buf.err_checked = True
@@ -285,6 +292,10 @@ class _Program:
                     src, dst, flags = outs[i - 1], outs[i], flags | 1
                 hip.call("tedq_jit_pass", fns[i], 0, hip.ptr(src), hip.ptr(dst), B, self.n, self.plan.k, self.plan.r,
                          mask, zero, hip.ptr(mats), self.plan.mat_stride, None, 0, 0, None, flags, st)
+            elif self.plan.lift:
+                hip.call("tedq_sv_lift_pass", 2 * self.general[i], hip.ptr(psi), None, B, self.n, self.plan.k,
+                         self.plan.r, tl, buf.pass_ptr(off), mask, zero, hip.ptr(mats), self.plan.mat_stride, None, 0,
+                         0, st)
             else:
                 hip.call("tedq_sv_apply_pass", hip.ptr(psi), B, self.n, self.plan.k, self.plan.r, tl,
                          buf.pass_ptr(off), mask, zero, hip.ptr(mats), self.plan.mat_stride, st)
@@ -328,6 +339,10 @@ class _Program:
                 hip.call("tedq_jit_pass", fn, 1, hip.ptr(src), hip.ptr(lam), B, self.n, self.plan.k, self.plan.r,
                          mask, zero, hip.ptr(mats), self.plan.mat_stride, hip.ptr(partials), rows, G, dy, flags,
                          st)
+            elif self.plan.lift:
+                hip.call("tedq_sv_lift_pass", 1 + 2 * self.general[P - 1 - i], hip.ptr(psi), hip.ptr(lam), B, self.n,
+                         self.plan.k, self.plan.r, tl, buf.pass_ptr(off), mask, zero, hip.ptr(mats),
+                         self.plan.mat_stride, hip.ptr(partials), rows, G, st)
             else:
                 hip.call("tedq_sv_adjoint_pass", hip.ptr(psi), hip.ptr(lam), B, self.n, self.plan.k, self.plan.r,
                          tl, buf.pass_ptr(off), mask, zero, hip.ptr(mats), self.plan.mat_stride,
@@ -405,8 +420,8 @@ class SVExecutor:
         device = device or torch.device("cuda", torch.cuda.current_device())
         if forward:
             k, r = self.fwd.plan.k, self.fwd.plan.r
-            if self.phase_free and jit.supported(self.n, k, r, False):
-                self.fwd = self._program(k, r, specialize=True)
+            if jit.supported(self.n, k, r, False):
+                self.fwd = self._program(k, r, specialize=self.phase_free)
             self.fwd.enable_jit(device, True, False)
         if adjoint:
             k, r = self.bwd.plan.k, self.bwd.plan.r
@@ -429,16 +444,17 @@ class SVExecutor:
             self.enable_jit(device)
             self._jitted.add(key)
 
-    def _program(self, k, r, specialize=False):
+    def _program(self, k, r, specialize=False, lift=False):
         """Fusion plan for (k, r), built once per executor (with its compiled kernels, if any).  The
         specialised plan keeps trainable rotations unfused (single-value gradients, real 2x2 ops) and
-        applies diagonal gates without their global phase, for generated kernels."""
+        applies diagonal gates without their global phase, for generated kernels; the lifted plan is the
+        interpreted kernels' form of it (planner.build_plan)."""
         if not hasattr(self, "_programs"):
             self._programs = {}
-        key = (k, r, specialize)
+        key = (k, r, specialize, lift)
         if key not in self._programs:
             self._programs[key] = _Program(self.n, self._units, self.n_params, list(self._pool), k, r,
-                                           specialize=specialize)
+                                           specialize=specialize, lift=lift)
         return self._programs[key]
 
     def configure(self, k, r, k_bwd=None, r_bwd=None):
@@ -447,8 +463,10 @@ class SVExecutor:
         k_bwd = k if k_bwd is None else k_bwd
         # the adjoint holds psi and lambda registers: more than 16 amplitudes each would spill
         r_bwd = min(4, r if r_bwd is None else r_bwd)
-        self.fwd = self._program(k, r)
-        self.bwd = self._program(k_bwd, r_bwd)
+        # lifted plans drop global phases: any adjoint sweep may (psi and lambda carry the same ones), the
+        # forward where no output shows them
+        self.fwd = self._program(k, r, lift="fwd" if self.phase_free else False)
+        self.bwd = self._program(k_bwd, r_bwd, lift=True)
         if self.jit:
             self._ensure_jit(torch.device("cuda", torch.cuda.current_device()))
 
@@ -501,7 +519,7 @@ class SVExecutor:
         phases), but an exact forward's checkpoints would meet a lambda whose phases differ."""
         f, b = self.fwd, self.bwd
         return (len(f.plan.passes) >= 2 and f.enc.tile_masks == b.enc.tile_masks
-                and f.plan.specialize == b.plan.specialize)
+                and f.plan.specialize == b.plan.specialize and f.plan.lift == b.plan.lift)
 
     def run_forward(self, params, need_grad=False):
         """Apply the circuit to every parameter row.  Returns psi [B, 2^n] complex64.
