@@ -259,6 +259,32 @@ int tedq_tn_gate_backward(const void* ec, int64_t ec_bstride, const void* x, int
                           int64_t g_bstride, void* ex, int64_t ex_bstride, void* eg, int64_t eg_bstride,
                           int64_t batch, const int32_t* desc, const int32_t* desc_dev, void* workspace,
                           int64_t workspace_bytes, void* stream);
+/* Chains of gate steps on one large tensor, a tile of address bits at a time
+ * (replaces runs of the pairwise steps of tree.contract,
+ * pytorch_backend.py:276-354).  ops: 52 int32 words per op = {arity 2 or 3,
+ * 3 slots, mask of the bits that go straight through, internal index count,
+ * factor count, matrix offset in coef, environment base (-1 none, 0, 1) and
+ * offset, 2 reserved, per factor {base, offset, rank, per address bit the
+ * variable it follows: 0..2 in, 3..5 out, 6..8 internal, 1 reserved}}, host and
+ * device copies.  plan: 128 int32 words per pass = {tile bits, outer bits, ops,
+ * matrix entries, [4..16) input address bit of every slot, [16..28) slot and
+ * [28..40) address bit of the tile's result bits, [40..60) and [72..92) input
+ * and result address bits of the outer bits}.  tedq_tn_run_coefs forms the
+ * matrices, tedq_tn_run_pass applies a pass (x and c distinct), and
+ * tedq_tn_run_backward undoes it from its result c (unitary matrices):
+ * environment ec of the result -> ex of the input (ex may be ec when the
+ * layout does not change), gate environments into env0 / env1. */
+int tedq_tn_run_coefs(const void* const* bases, const int64_t* strides, const int64_t* lens, const int32_t* ops,
+                      const int32_t* ops_dev, int n_ops, void* coef, int64_t coef_bstride, int64_t batch,
+                      void* stream);
+int tedq_tn_run_pass(const void* x, int64_t x_bstride, void* c, int64_t c_bstride, int64_t batch, const int32_t* plan,
+                     const int32_t* ops, const int32_t* ops_dev, const void* coef, int64_t coef_bstride, void* stream);
+int64_t tedq_tn_run_backward_workspace(const int32_t* plan, int64_t batch);
+int tedq_tn_run_backward(const void* c, int64_t c_bstride, const void* ec, int64_t ec_bstride, void* ex,
+                         int64_t ex_bstride, int64_t batch, const int32_t* plan, const int32_t* ops,
+                         const int32_t* ops_dev, const void* coef, int64_t coef_bstride, void* env0,
+                         int64_t env0_bstride, int64_t env0_len, void* env1, int64_t env1_bstride, int64_t env1_len,
+                         void* workspace, int64_t workspace_bytes, void* stream);
 /* Gate tensors of the network's leaves for every parameter row: ket U with
  * axes (out..., in...) or bra U^dagger, and dV/dtheta 2x2 blocks of trainable
  * parameters.  recs: dev int32[16] records {code, src0..2, const_off, nq,

@@ -58,6 +58,11 @@ _SIGNATURES = {
     "tedq_tn_gate_backward_workspace": ([c_vp, c_i64], c_i64),
     "tedq_tn_gate_backward": ([c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_i64, c_vp, c_vp,
                                c_vp, c_i64, c_vp], c_int),
+    "tedq_tn_run_coefs": ([c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_vp, c_i64, c_i64, c_vp], c_int),
+    "tedq_tn_run_pass": ([c_vp, c_i64, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp], c_int),
+    "tedq_tn_run_backward_workspace": ([c_vp, c_i64], c_i64),
+    "tedq_tn_run_backward": ([c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_i64,
+                              c_i64, c_vp, c_i64, c_i64, c_vp, c_i64, c_vp], c_int),
     "tedq_tn_gate_tensors": ([c_vp, c_int, c_i64, c_int, c_vp, c_int, c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_vp],
                              c_int),
     "tedq_tn_param_grad": ([c_vp, c_i64, c_vp, c_i64, c_vp, c_int, c_vp, c_vp, c_i64, c_vp], c_int),

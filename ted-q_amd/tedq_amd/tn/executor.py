@@ -18,6 +18,9 @@ What is this module's own:
 * each pairwise step is one tedq_tn_contract launch over the whole parameter
   batch, reading operands and writing the result through index-bit layouts
   (no permuted copies);
+* chains of gate-sized tensors on one large intermediate run as passes over
+  LDS tiles (``runs``): the intermediate crosses HBM once per pass instead of
+  once per gate, forward and backward;
 * gradients come from the reverse contraction tree: the environment of a
   step's result gives the environments of its two operands (two more
   contraction launches), and the environments of the gate leaves give
@@ -37,6 +40,7 @@ import torch
 from ..engine import hip
 from ..engine.sv import MeasSpec, check_device_flag
 from ..measurement import Expectation, Probability, State
+from . import runs as R
 from .network import cancel_inverse_pairs, diagonal_reduce
 from .path import external_path, path_sets, path_stats, search_path
 from .slicing import choose_slices, slice_network
@@ -81,6 +85,19 @@ def diagonal_wires(op):
     if op.num_params == 0:
         return _leading_diagonal_wires(op.matrix, nq)
     return 0
+
+
+def _unitary_matrix(m):
+    m = np.asarray(m, dtype=np.complex128)
+    m = m.reshape(int(round(np.sqrt(m.size))), -1)
+    return bool(np.max(np.abs(m @ m.conj().T - np.eye(m.shape[0]))) < 1e-6)
+
+
+def _unitary_gate(op):
+    """Parametrised gates are unitary for every value; a constant matrix is what the user gave."""
+    return op.num_params > 0 or _unitary_matrix(op.matrix)
+
+
 _NO_SRC = -2 ** 31
 _DESC_WORDS = 4 + 9 * 32
 _ROLE = {"AH": 0, "AM": 1, "AK": 2, "BH": 3, "BK": 4, "BN": 5, "CH": 6, "CM": 7, "CN": 8}
@@ -355,7 +372,11 @@ class TNExecutor:
         self.small_batch = True
         # backward: both environments of a gate step from one pass (tedq_tn_gate_backward)
         self.fused_backward = True
+        # chains of gates on one large tensor as passes over LDS tiles (tedq_tn_run_pass / _backward)
+        self.run_passes = True
         self._small = {}
+        self._run_plans = {}
+        self._leaf_unitary = {idx: _unitary_gate(op) for idx, op in cc._operators.items()}  # pylint: disable=protected-access
         ext = _external_paths(cc, paths)
         # diagonal reduction (the reference's tn_simplify, by gate type): the wires along which gates are
         # diagonal (all of a diagonal gate's, the controls of a controlled gate) are merged into
@@ -634,6 +655,113 @@ class TNExecutor:
         self._small[key] = plan
         return plan
 
+    # runs of gates on one large tensor ------------------------------------
+    def _use_runs(self, dev):
+        """Runs are a device path: they need the small steps' results in their arena."""
+        return self.run_passes and self.small_batch and dev.type == "cuda"
+
+    def _run_plan(self, net, grad):
+        """The network's runs (``grad``: those the backward can undo), their op table and pass words."""
+        key = (id(net), grad)
+        if key in self._run_plans:
+            return self._run_plans[key]
+        small = self._small_plan(net)
+        offs = small["offs"]
+
+        def leaf_unitary(source, rank):
+            if source[0] in ("gate", "adj"):
+                return self._leaf_unitary[source[1]]
+            if source[0] == "obs":
+                m = np.asarray(net.measurement.obs[source[1]].matrix)
+            elif source[0] == "obsmat":
+                m = np.asarray(net.measurement.obs.matrix)
+            else:
+                return False
+            return m.size == 1 << rank and _unitary_matrix(m)
+
+        def source(tid):
+            if tid < net.n_inputs:
+                where, o = net.leaves[tid]
+                return (0 if where == "arena" else 1), o
+            return 2, offs[tid]
+
+        found = R.find_runs(net, offs, grad, R.Unitarity(net, leaf_unitary) if grad else None)
+        rows, coef = [], 0
+        for run in found:
+            enc = R.encode_run(run, source, net.lay)
+            for ps in run.passes:
+                ps.head = len(rows)
+                for op in ps.ops:
+                    w = enc.pop(0)
+                    w[7] += coef
+                    tid = op.factors[0]
+                    base, o = source(tid)
+                    w[8], w[9] = (-1, 0) if base == 1 or not net.needs[tid] else (0 if base == 0 else 1, o)
+                    rows.append(w)
+                coef += int(ps.words[3])
+        plan = {"first": {run.steps[0]: run for run in found}, "last": {run.steps[-1]: run for run in found},
+                "covered": {s for run in found for s in run.steps},
+                "ops": np.array(rows, dtype=np.int32).reshape(-1, R.OP_WORDS), "coef": coef, "dev": {}}
+        self._run_plans[key] = plan
+        return plan
+
+    def _run_coefs(self, plan, small, arena, leaves, buf, B, dev):
+        """The op matrices of every run of a network, one launch: [B, plan coef]."""
+        key = str(dev)
+        if key not in plan["dev"]:
+            plan["dev"][key] = torch.from_numpy(plan["ops"].reshape(-1).copy()).to(dev)
+        consts = buf["consts"]
+        coef = torch.empty((B, plan["coef"]), dtype=torch.complex64, device=dev)
+        bases = (ctypes.c_void_p * 3)(leaves.data_ptr(), consts.data_ptr(), arena.data_ptr())
+        strides = (ctypes.c_int64 * 3)(self.leaf_stride, 0, small["len"])
+        lens = (ctypes.c_int64 * 3)(self.leaf_stride, consts.numel(), small["len"])
+        hip.call("tedq_tn_run_coefs", bases, strides, lens, plan["ops"].ctypes.data_as(hip.c_vp),
+                 hip.ptr(plan["dev"][key]), len(plan["ops"]), hip.ptr(coef), plan["coef"], B, hip.stream_handle(dev))
+        return coef
+
+    @staticmethod
+    def _op_rows(plan, ps, dev):
+        return (ctypes.c_void_p(plan["ops"].ctypes.data + 4 * R.OP_WORDS * ps.head),
+                ctypes.c_void_p(plan["dev"][str(dev)].data_ptr() + 4 * R.OP_WORDS * ps.head))
+
+    def _run_forward_passes(self, run, plan, coef, x, B, dev, keep):
+        """The results of a run's passes (only the last one unless ``keep``)."""
+        outs = []
+        spare = None
+        for i, ps in enumerate(run.passes):
+            out = spare
+            if out is None or keep or i == len(run.passes) - 1:
+                out = torch.empty((B, 1 << run.wires), dtype=torch.complex64, device=dev)
+            hip.call("tedq_tn_run_pass", ctypes.c_void_p(x[0].data_ptr() + 8 * x[2]), x[1], hip.ptr(out), out.shape[1],
+                     B, ps.words.ctypes.data_as(hip.c_vp), *self._op_rows(plan, ps, dev), hip.ptr(coef),
+                     plan["coef"], hip.stream_handle(dev))
+            spare = x[0] if i > 0 and not keep else None
+            x = (out, out.shape[1], 0)
+            outs.append(out)
+        return outs if keep else outs[-1:]
+
+    def _run_backward_passes(self, run, plan, coef, outs, env, env_arena, env_small, B, dev):
+        """Environment of a run's input from its result's, the gates' environments going to the arenas."""
+        lib = hip.load()
+        owned = False
+        for i in range(len(run.passes) - 1, -1, -1):
+            ps, c = run.passes[i], outs[i]
+            words = ps.words.ctypes.data_as(hip.c_vp)
+            ws_bytes = lib.tedq_tn_run_backward_workspace(words, B)
+            if ws_bytes < 0:
+                raise hip.EngineError("tensor network: invalid run pass")
+            ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
+            ex = env[0] if owned else torch.empty((B, 1 << run.wires), dtype=torch.complex64, device=dev)
+            hip.call("tedq_tn_run_backward", hip.ptr(c), c.shape[1],
+                     ctypes.c_void_p(env[0].data_ptr() + 8 * env[2]), env[1], hip.ptr(ex), ex.shape[1], B, words,
+                     *self._op_rows(plan, ps, dev), hip.ptr(coef), plan["coef"], hip.ptr(env_arena),
+                     self.leaf_stride, self.leaf_stride, hip.ptr(env_small), env_small.shape[1], env_small.shape[1],
+                     hip.ptr(ws), ws_bytes, hip.stream_handle(dev))
+            # only the last pass changes the layout, so the others may write over the environment they read
+            owned = True
+            env = (ex, ex.shape[1], 0)
+        return env[0]
+
     def _small_levels(self, plan, arena, leaves, buf, B, dev):
         """Run a plan's levels in order, one launch each, results into ``arena`` [B, plan len]."""
         key = str(dev)
@@ -710,11 +838,17 @@ class TNExecutor:
             return total, {}
         return self._forward_once(net, leaves, B, dev, keep)
 
-    def _forward_once(self, net, leaves, B, dev, keep=None):
+    def _forward_once(self, net, leaves, B, dev, keep=None, grad_runs=False):
+        """``keep`` None: forward only, with every run of the network; else the steps one by one, or with
+        ``grad_runs`` the runs that the backward undoes (their matrices and pass results go to ``kept``)."""
         buf = self._buffers(dev)
         vals = {}
         kept = {}
         small = self._small_plan(net) if self.small_batch else None
+        plan = self._run_plan(net, grad_runs) if (keep is None or grad_runs) and self._use_runs(dev) else None
+        if plan is not None and not plan["first"]:
+            plan = None
+        arena = leaves
         if small is not None and small["bounds"]:
             arena = torch.empty((B, small["len"]), dtype=torch.complex64, device=dev)
             self._small_levels(small, arena, leaves, buf, B, dev)
@@ -722,8 +856,21 @@ class TNExecutor:
                 vals[tid] = (arena, small["len"], o)
                 if keep is not None and tid != net.root and keep(tid):
                     kept[tid] = vals[tid]
-        for st in net.steps:
+        coef = self._run_coefs(plan, small, arena, leaves, buf, B, dev) if plan is not None else None
+        if grad_runs:
+            kept["coef"] = coef
+        for s, st in enumerate(net.steps):
             if small is not None and st.c in small["offs"]:
+                continue
+            if plan is not None and s in plan["covered"]:
+                run = plan["first"].get(s)
+                if run is not None:
+                    outs = self._run_forward_passes(run, plan, coef, self._operand(net, vals, run.a, leaves, buf), B,
+                                                    dev, grad_runs)
+                    vals[run.c] = outs[-1]
+                    if grad_runs:
+                        kept["run", s] = outs
+                    vals.pop(run.a, None)
                 continue
             out = torch.empty((B, 1 << net.ranks[st.c]), dtype=torch.complex64, device=dev)
             vals[st.c] = out
@@ -780,6 +927,12 @@ class TNExecutor:
         seg = max(1, int(math.ceil(math.sqrt(len(net.steps)))))
         return [list(range(s, min(s + seg, len(net.steps)))) for s in range(0, len(net.steps), seg)]
 
+    def _run_bytes(self, net, plan, B):
+        """Bytes of intermediates the backward keeps when the runs store one tensor per pass."""
+        elems = sum(len(run.passes) << run.wires for run in plan["first"].values())
+        elems += sum(1 << net.ranks[st.c] for s, st in enumerate(net.steps) if s not in plan["covered"])
+        return elems * B * 8
+
     def _backward_network(self, net, leaves, dmats, root_env, grad, B, dev):
         """Reverse contraction tree of one network; gradients are added into ``grad``.  Returns the
         network's root.  A sliced network runs forward and backward once per slice: the parameter
@@ -795,7 +948,10 @@ class TNExecutor:
 
     def _backward_once(self, net, leaves, dmats, root_env, grad, B, dev):
         buf = self._buffers(dev)
-        segs = self._segments(net, B, dev)
+        plan = self._run_plan(net, True) if self._use_runs(dev) else None
+        if plan is not None and (not plan["first"] or self._run_bytes(net, plan, B) > self._keep_budget(dev)):
+            plan = None
+        segs = [list(range(len(net.steps)))] if plan is not None else self._segments(net, B, dev)
         seg_of = {}
         for si, seg in enumerate(segs):
             for s in seg:
@@ -807,7 +963,12 @@ class TNExecutor:
         else:
             def keep(t):
                 return seg_of.get(t, -1) != seg_of.get(net.steps[net.consumer[t]].c, -1)
-        root, stored = self._forward_once(net, leaves, B, dev, keep)
+        root, stored = self._forward_once(net, leaves, B, dev, keep, plan is not None)
+        coef = stored.pop("coef", None)
+        env_small = None
+        if plan is not None:
+            small = self._small_plan(net)
+            env_small = torch.zeros((B, small["len"]), dtype=torch.complex64, device=dev)
         env_arena = torch.zeros((B, self.leaf_stride), dtype=torch.complex64, device=dev)
         envs = {net.root: root_env}
         for si in range(len(segs) - 1, -1, -1):
@@ -826,10 +987,25 @@ class TNExecutor:
                                    buf)
             for s in reversed(seg):
                 st = net.steps[s]
+                if plan is not None and s in plan["covered"]:
+                    run = plan["last"].get(s)
+                    if run is not None:
+                        outs = stored.pop(("run", run.steps[0]))
+                        vals.pop(("run", run.steps[0]), None)
+                        vals.pop(run.c, None)
+                        e = envs.pop(run.c, None)
+                        if e is None:
+                            continue
+                        e = e if isinstance(e, tuple) else (e, e.shape[1], 0)
+                        envs[run.a] = self._run_backward_passes(run, plan, coef, outs, e, env_arena, env_small, B, dev)
+                        for t in (t for ps in run.passes for op in ps.ops for t in op.factors):
+                            if t >= net.n_inputs and net.needs[t]:
+                                envs[t] = (env_small, env_small.shape[1], small["offs"][t])
+                    continue
                 ec = envs.pop(st.c, None)
                 if ec is None:
                     continue
-                ecop = (ec, ec.shape[1], 0)
+                ecop = ec if isinstance(ec, tuple) else (ec, ec.shape[1], 0)
                 dsts = {}
                 for which, desc_row, tid in (("a", st.bwd_a, st.a), ("b", st.bwd_b, st.b)):
                     if desc_row < 0:
