@@ -143,6 +143,20 @@ int tedq_sv_lambda_z(const void* psi, void* lam, int64_t batch, int n_qubits, co
  * (pytorch_backend.py:402-424, 428-459). */
 int tedq_sv_expval_factored(const void* state, int64_t batch, int n_qubits, int q, const int* bits,
                             const float* factors, uint64_t zmask, double* partial, double* out, void* stream);
+/* The same for count observables of q factors each in one launch: records =
+ * count records of tedq_sv_factored_record_bytes() bytes, filled by
+ * tedq_sv_factored_record (host) and an identical device copy; partial: dev
+ * double [batch][count][tedq_sv_factored_chunks(n, q)]; out: dev double [batch][count]. */
+int64_t tedq_sv_factored_record_bytes(void);
+int tedq_sv_factored_record(void* record, int n_qubits, int q, const int* bits, const float* factors,
+                            uint64_t zmask);
+int64_t tedq_sv_factored_chunks(int n_qubits, int q);
+int tedq_sv_expval_factored_batch(const void* state, int64_t batch, int n_qubits, int q, const void* records,
+                                  const void* records_dev, int count, double* partial, double* out, void* stream);
+/* lam += sum over count one-factor observables of coef[b][o] Zsign_o ((F_o + F_o^dagger)/2) psi
+ * (coef: dev double [batch][count]). */
+int tedq_sv_lambda_factored_batch(const void* psi, void* lam, int64_t batch, int n_qubits, const void* records,
+                                  const void* records_dev, int count, const double* coef, void* stream);
 /* lam += coef[b] * Zsign * ((F + F^dagger)/2) psi  (coef: dev double [batch]). */
 int tedq_sv_lambda_factored(const void* psi, void* lam, int64_t batch, int n_qubits, int q, const int* bits,
                             const float* factors, uint64_t zmask, const double* coef, void* stream);

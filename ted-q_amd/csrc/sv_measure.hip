@@ -6,6 +6,8 @@
 // Here all diagonal (Z-string) observables of a circuit are reduced in ONE
 // pass, accumulated in fp64 per thread and combined across workgroups with
 // Neumaier-compensated fp64 summation; the mask 0 observable is the norm.
+#include <string.h>
+
 #include <mutex>
 
 #include "tedq_common.h"
@@ -173,6 +175,58 @@ __global__ void k_sum_partials(const double* __restrict__ partial, int64_t batch
   out[i] = (OT)(s + c);
 }
 
+// The same sums for many chunks: a workgroup owns 2^ml adjacent columns m of
+// one b and spreads the chunks over its threads (each a compensated sum over a
+// fixed stride, then a fixed order over the threads), because a thread per
+// output is a chain of nchunk dependent loads: 265 us for 1024 chunks of 25
+// columns, 15 us here.
+constexpr int kWideSumChunks = 16;
+
+template <typename OT>
+__global__ void __launch_bounds__(kRedThreads) k_sum_partials_wide(const double* __restrict__ partial, int64_t nchunk,
+                                                                   int M, int ml, int64_t mtiles,
+                                                                   OT* __restrict__ out) {
+  __shared__ double rs[kRedThreads], rc[kRedThreads];
+  const int64_t b = blockIdx.x / mtiles;
+  const int64_t m = ((blockIdx.x - b * mtiles) << ml) + (threadIdx.x & ((1 << ml) - 1));
+  const int step = kRedThreads >> ml;
+  double s = 0.0, c = 0.0;
+  if (m < M)
+#pragma unroll 4
+    for (int64_t ch = threadIdx.x >> ml; ch < nchunk; ch += step) neumaier(s, c, partial[(b * nchunk + ch) * M + m]);
+  rs[threadIdx.x] = s;
+  rc[threadIdx.x] = c;
+  for (int h = step >> 1; h > 0; h >>= 1) {
+    __syncthreads();
+    if ((threadIdx.x >> ml) < h) {
+      const int o = threadIdx.x + (h << ml);
+      neumaier(s, c, rs[o]);
+      c += rc[o];
+      rs[threadIdx.x] = s;
+      rc[threadIdx.x] = c;
+    }
+  }
+  if (m < M && threadIdx.x < (1 << ml)) out[b * M + m] = (OT)(s + c);
+}
+
+// Chunk sums, both forms: few chunks leave the wide one's threads idle, so a thread per output is kept
+// below 16 (1 to 8 chunks: 4 us either way).
+template <typename OT>
+static void sum_partials(const double* partial, int64_t batch, int64_t nchunk, int64_t M, OT* out, hipStream_t st) {
+  if (nchunk >= kWideSumChunks) {
+    int ml = 0;
+    while (ml < 5 && (1 << ml) < M) ++ml;
+    const int64_t mtiles = (M + (1 << ml) - 1) >> ml;
+    if (batch * mtiles <= 0x7fffffffll) {
+      hipLaunchKernelGGL(k_sum_partials_wide<OT>, dim3((unsigned)(batch * mtiles)), dim3(kRedThreads), 0, st, partial,
+                         nchunk, (int)M, ml, mtiles, out);
+      return;
+    }
+  }
+  hipLaunchKernelGGL(k_sum_partials<OT>, dim3((unsigned)((batch * M + 127) / 128)), dim3(128), 0, st, partial, batch,
+                     nchunk, (int)M, out);
+}
+
 // lambda_x = (sum_m dy[b][m] (-1)^popc(x & mask_m)) psi_x      (M may be 0: lambda = 0)
 __global__ void k_lambda_z(const float2* __restrict__ psi, float2* __restrict__ lam, int64_t total, int n,
                            const uint64_t* __restrict__ masks, int M, const double* __restrict__ dy) {
@@ -239,12 +293,15 @@ __global__ void __launch_bounds__(kRedThreads) k_lambda_z_wht(const float2* __re
 struct FactorObs {
   int q;
   int bits[4];        // physical positions
+  int sorted[4];      // the same, ascending
   float2 f[4][4];     // 2x2 factor per bit, row-major
   uint64_t zmask;
 };
 
-__device__ __forceinline__ void apply_factors(float2 (&g)[16], const FactorObs& o, bool dagger) {
-  for (int t = 0; t < o.q; ++t) {
+template <int Q>
+__device__ __forceinline__ void apply_factors(float2 (&g)[1 << Q], const FactorObs& o, bool dagger) {
+#pragma unroll
+  for (int t = 0; t < Q; ++t) {
     float2 m0 = o.f[t][0], m1 = o.f[t][1], m2 = o.f[t][2], m3 = o.f[t][3];
     if (dagger) {
       const float2 tmp = m1;
@@ -253,8 +310,8 @@ __device__ __forceinline__ void apply_factors(float2 (&g)[16], const FactorObs& 
       m2 = cconj(tmp);
       m3 = cconj(m3);
     }
-    const int sz = 1 << o.q;
-    for (int i = 0; i < sz; ++i) {
+#pragma unroll
+    for (int i = 0; i < (1 << Q); ++i) {
       if (i & (1 << t)) continue;
       const int j = i | (1 << t);
       const float2 x = g[i], y = g[j];
@@ -264,51 +321,58 @@ __device__ __forceinline__ void apply_factors(float2 (&g)[16], const FactorObs& 
   }
 }
 
-__device__ __forceinline__ uint64_t group_index(uint64_t gid, const FactorObs& o, int t) {
-  // insert the bits of t (bit i -> physical o.bits[i]) into gid with zeros at o.bits
-  uint64_t x = gid;
-  // bits must be inserted in ascending physical order
-  int order[4];
-  for (int i = 0; i < o.q; ++i) order[i] = i;
-  for (int i = 0; i < o.q; ++i)
-    for (int j = i + 1; j < o.q; ++j)
-      if (o.bits[order[j]] < o.bits[order[i]]) {
-        const int tmp = order[i];
-        order[i] = order[j];
-        order[j] = tmp;
-      }
-  for (int ii = 0; ii < o.q; ++ii) {
-    const int p = o.bits[order[ii]];
-    const uint64_t low = x & ((1ull << p) - 1);
-    x = ((x >> p) << (p + 1)) | low;
+// amplitude of group gid with the observable's bits clear
+template <int Q>
+__device__ __forceinline__ uint64_t group_base(uint64_t gid, const FactorObs& o) {
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const int p = o.sorted[i];
+    gid = ((gid >> p) << (p + 1)) | (gid & ((1ull << p) - 1));
   }
-  for (int i = 0; i < o.q; ++i)
+  return gid;
+}
+
+template <int Q>
+__device__ __forceinline__ uint64_t group_bits(int t, const FactorObs& o) {
+  uint64_t x = 0;
+#pragma unroll
+  for (int i = 0; i < Q; ++i)
     if ((t >> i) & 1) x |= 1ull << o.bits[i];
   return x;
 }
 
-__global__ void __launch_bounds__(kRedThreads) k_expval_factored(const float2* __restrict__ st, int n, FactorObs o,
-                                                                  double* __restrict__ partial, int64_t ngroups,
-                                                                  int64_t nchunk) {
+// Observables of one kind (Q bits), all of a circuit's in one launch: workgroup
+// (chunk, b, o) sums groups [chunk * per, + per) into partial[b][o][chunk].
+// Bound by latency at small sizes: one launch per observable with one chunk of
+// 2^14 amplitudes per workgroup ran 15 observables of 16 x 2^15 amplitudes in
+// 15 x 46 us (32 workgroups each, the group arrays in scratch memory); with
+// the observables and chunks of 2^11 groups in the grid and the arrays in
+// registers it is 9 us for all of them.
+template <int Q>
+__global__ void __launch_bounds__(kRedThreads) k_expval_factored(const float2* __restrict__ st, int n,
+                                                                  const FactorObs* __restrict__ obs, FactorObs one,
+                                                                  double* __restrict__ partial, int64_t per) {
   __shared__ double red[kRedThreads / 64];
+  const FactorObs o = obs != nullptr ? obs[blockIdx.z] : one;
   const int64_t b = blockIdx.y;
   const float2* s = st + (b << n);
-  const int64_t per = (ngroups + nchunk - 1) / nchunk;
+  const int64_t ngroups = 1ll << (n - Q);
   const int64_t g0 = blockIdx.x * per, g1 = g0 + per < ngroups ? g0 + per : ngroups;
   double acc = 0.0;
-  const int sz = 1 << o.q;
+#pragma unroll(Q <= 1 ? 4 : 1)
   for (int64_t gid = g0 + threadIdx.x; gid < g1; gid += kRedThreads) {
-    float2 g[16], h[16];
-    uint64_t idx[16];
-    for (int t = 0; t < sz; ++t) {
-      idx[t] = group_index((uint64_t)gid, o, t);
-      g[t] = s[idx[t]];
+    float2 g[1 << Q], h[1 << Q];
+    const uint64_t base = group_base<Q>((uint64_t)gid, o);
+#pragma unroll
+    for (int t = 0; t < (1 << Q); ++t) {
+      g[t] = s[base | group_bits<Q>(t, o)];
       h[t] = g[t];
     }
-    apply_factors(h, o, false);
-    const double zs = (__popcll(idx[0] & o.zmask) & 1) ? -1.0 : 1.0;
+    apply_factors<Q>(h, o, false);
+    const double zs = (__popcll(base & o.zmask) & 1) ? -1.0 : 1.0;
     double part = 0.0;
-    for (int t = 0; t < sz; ++t) part += (double)g[t].x * h[t].x + (double)g[t].y * h[t].y;
+#pragma unroll
+    for (int t = 0; t < (1 << Q); ++t) part += (double)g[t].x * h[t].x + (double)g[t].y * h[t].y;
     acc += zs * part;
   }
   acc = wave_sum_d(acc);
@@ -317,11 +381,47 @@ __global__ void __launch_bounds__(kRedThreads) k_expval_factored(const float2* _
   if (threadIdx.x == 0) {
     double t = 0.0;
     for (int w = 0; w < kRedThreads / 64; ++w) t += red[w];
-    partial[b * nchunk + blockIdx.x] = t;
+    partial[(b * gridDim.z + blockIdx.z) * gridDim.x + blockIdx.x] = t;
   }
 }
 
+// lambda += sum_o coef[b][o] * zsign_o * ((F_o + F_o^dagger)/2) psi for all
+// one-bit observables of a circuit: a thread per amplitude adds the terms in
+// the observables' order, so lambda is read and written once instead of once
+// per observable (15 x 9 us -> 14 us at 16 x 2^15 amplitudes); the partner
+// amplitudes come from cache.
+__global__ void __launch_bounds__(256) k_lambda_factored1(const float2* __restrict__ psi, float2* __restrict__ lam,
+                                                          int n, const FactorObs* __restrict__ obs, int count,
+                                                          const double* __restrict__ coef, int64_t total) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const int64_t b = i >> n;
+  const uint64_t x = (uint64_t)i & ((1ull << n) - 1);
+  const float2 p = psi[i];
+  float2 cur = lam[i];
+  for (int k = 0; k < count; ++k) {
+    const FactorObs& o = obs[k];
+    const uint64_t bit = 1ull << o.bits[0];
+    const float2 y = psi[(b << n) | (int64_t)(x ^ bit)];
+    const float2 m0 = o.f[0][0], m1 = o.f[0][1], m2 = o.f[0][2], m3 = o.f[0][3];
+    const double zs = (__popcll(x & ~bit & o.zmask) & 1) ? -1.0 : 1.0;
+    const float c = (float)(0.5 * zs * coef[b * count + k]);
+    float2 h1, h2;
+    if (x & bit) {
+      h1 = cmul2(m2, y, m3, p);
+      h2 = cmul2(cconj(m1), y, cconj(m3), p);
+    } else {
+      h1 = cmul2(m0, p, m1, y);
+      h2 = cmul2(cconj(m0), p, cconj(m2), y);
+    }
+    cur.x += c * (h1.x + h2.x);
+    cur.y += c * (h1.y + h2.y);
+  }
+  lam[i] = cur;
+}
+
 // lambda += coef[b] * zsign * ((F + F^dagger)/2) psi on every group
+template <int Q>
 __global__ void k_lambda_factored(const float2* __restrict__ psi, float2* __restrict__ lam, int n, FactorObs o,
                                   int64_t ngroups, const double* __restrict__ coef, int64_t batch) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -329,24 +429,22 @@ __global__ void k_lambda_factored(const float2* __restrict__ psi, float2* __rest
   const int64_t b = i / ngroups, gid = i - b * ngroups;
   const float2* s = psi + (b << n);
   float2* l = lam + (b << n);
-  const int sz = 1 << o.q;
-  float2 g[16], h1[16], h2[16];
-  uint64_t idx[16];
-  for (int t = 0; t < sz; ++t) {
-    idx[t] = group_index((uint64_t)gid, o, t);
-    g[t] = s[idx[t]];
-    h1[t] = g[t];
-    h2[t] = g[t];
+  float2 h1[1 << Q], h2[1 << Q];
+  const uint64_t base = group_base<Q>((uint64_t)gid, o);
+#pragma unroll
+  for (int t = 0; t < (1 << Q); ++t) {
+    h1[t] = s[base | group_bits<Q>(t, o)];
+    h2[t] = h1[t];
   }
-  apply_factors(h1, o, false);
-  apply_factors(h2, o, true);
-  const double zs = (__popcll(idx[0] & o.zmask) & 1) ? -1.0 : 1.0;
+  apply_factors<Q>(h1, o, false);
+  apply_factors<Q>(h2, o, true);
+  const double zs = (__popcll(base & o.zmask) & 1) ? -1.0 : 1.0;
   const float c = (float)(0.5 * zs * coef[b]);
-  for (int t = 0; t < sz; ++t) {
-    float2 cur = l[idx[t]];
+#pragma unroll
+  for (int t = 0; t < (1 << Q); ++t) {
+    float2& cur = l[base | group_bits<Q>(t, o)];
     cur.x += c * (h1[t].x + h2[t].x);
     cur.y += c * (h1[t].y + h2[t].y);
-    l[idx[t]] = cur;
   }
 }
 
@@ -381,7 +479,9 @@ __device__ __forceinline__ uint64_t deposit_outcome(uint32_t y, const BitList& b
 // Marginal probabilities without atomics, so the summation order is fixed.
 // Block (bin * nrc + rc, b) sums |psi_x|^2 in fp64 over 2^clog values r of the
 // remaining bits (clog = min(n - k, 14), r in rest chunk rc) of outcome bin, by
-// a fixed per-thread stride and a fixed tree, into partial[b][rc][bin].
+// a fixed per-thread stride and a fixed tree, into partial[b][rc][bin].  8 x 2^18
+// amplitudes, one bit: 15 us (60 us with a deposit of all bits per amplitude and
+// one load in flight).
 __global__ void __launch_bounds__(kRedThreads) k_probs_marg(const float2* __restrict__ st, int n, BitList bl,
                                                              uint64_t rest_mask, double* __restrict__ partial,
                                                              int64_t nrc) {
@@ -390,12 +490,28 @@ __global__ void __launch_bounds__(kRedThreads) k_probs_marg(const float2* __rest
   const int64_t bin = blockIdx.x / nrc, rc = blockIdx.x - bin * nrc;
   const int rest = n - bl.k;
   const int clog = rest < kChunkLog ? rest : kChunkLog;
-  const uint64_t fixed = deposit_outcome((uint32_t)bin, bl);
+  // the position of i = j * 256 + t is the union of the positions of rc, j and t: one deposit per
+  // thread for t and rc, four uniform ones for the bits of j, eight loads in flight
+  const uint64_t fixed = deposit_outcome((uint32_t)bin, bl) | pdep64((uint64_t)(rc << clog), rest_mask) |
+                         pdep64((uint64_t)threadIdx.x, rest_mask);
   const float2* base = st + (b << n);
   double acc = 0.0;
-  for (int64_t i = threadIdx.x; i < (1ll << clog); i += kRedThreads) {
-    const float2 a = base[fixed | pdep64((uint64_t)((rc << clog) + i), rest_mask)];
-    acc += (double)a.x * a.x + (double)a.y * a.y;
+  const int64_t count = 1ll << clog;
+  if (threadIdx.x < count) {
+    const int iters = (int)((count + kRedThreads - 1) / kRedThreads);
+    uint64_t low[3];
+#pragma unroll
+    for (int h = 0; h < 3; ++h) low[h] = pdep64((uint64_t)kRedThreads << h, rest_mask);
+    for (int j0 = 0; j0 < iters; j0 += 8) {
+      const uint64_t at = fixed | pdep64((uint64_t)j0 * kRedThreads, rest_mask);
+      float2 a[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j0 + j < iters) a[j] = base[at | (j & 1 ? low[0] : 0) | (j & 2 ? low[1] : 0) | (j & 4 ? low[2] : 0)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j0 + j < iters) acc += (double)a[j].x * a[j].x + (double)a[j].y * a[j].y;
+    }
   }
   acc = wave_sum_d(acc);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
@@ -555,8 +671,7 @@ static int launch_expval_z(const void* state, int64_t batch, int n_qubits, const
                        static_cast<const float2*>(state), n_qubits, dev_masks, n_masks, partial, nchunk);
   int rc = check_launch("tedq_sv_expval_z(partial)");
   if (rc) return rc;
-  hipLaunchKernelGGL(k_sum_partials<double>, dim3(nblocks(batch * n_masks, 128)), dim3(128), 0, st, partial, batch, nchunk,
-                     n_masks, out);
+  sum_partials(partial, batch, nchunk, n_masks, out, st);
   return check_launch("tedq_sv_expval_z(sum)");
 }
 
@@ -647,14 +762,43 @@ extern "C" int tedq_sv_lambda_z(const void* psi, void* lam, int64_t batch, int n
 static int make_factor_obs(FactorObs* o, int n, int q, const int* bits, const float* factors, uint64_t zmask) {
   if (q < 0 || q > 4) return kUnsupported;
   o->q = q;
-  for (int i = 0; i < 4; ++i) o->bits[i] = 0;
+  for (int i = 0; i < 4; ++i) o->bits[i] = o->sorted[i] = 0;
   for (int i = 0; i < q; ++i) {
     if (bits[i] < 0 || bits[i] >= n) return kBadArgument;
     o->bits[i] = bits[i];
+    int k = i;
+    for (; k > 0 && o->sorted[k - 1] > bits[i]; --k) o->sorted[k] = o->sorted[k - 1];
+    o->sorted[k] = bits[i];
     for (int j = 0; j < 4; ++j) o->f[i][j] = make_float2(factors[(i * 4 + j) * 2], factors[(i * 4 + j) * 2 + 1]);
   }
   o->zmask = zmask;
   return kOk;
+}
+
+#define TEDQ_FACTORED_CASES(LAUNCH) \
+  switch (q) {                      \
+    case 0: LAUNCH(0); break;       \
+    case 1: LAUNCH(1); break;       \
+    case 2: LAUNCH(2); break;       \
+    case 3: LAUNCH(3); break;       \
+    default: LAUNCH(4); break;      \
+  }
+
+static int launch_expval_factored(const void* state, int64_t batch, int n_qubits, int q, const FactorObs* obs,
+                                  const FactorObs& one, int count, int64_t nchunk, double* partial, double* out,
+                                  hipStream_t st) {
+  const int64_t ngroups = 1ll << (n_qubits - q);
+  const int64_t per = (ngroups + nchunk - 1) / nchunk;
+  const dim3 grid((unsigned)nchunk, (unsigned)batch, (unsigned)count);
+#define TEDQ_LAUNCH(Q)                                                                                            \
+  hipLaunchKernelGGL(k_expval_factored<Q>, grid, dim3(kRedThreads), 0, st, static_cast<const float2*>(state), n_qubits, \
+                     obs, one, partial, per)
+  TEDQ_FACTORED_CASES(TEDQ_LAUNCH)
+#undef TEDQ_LAUNCH
+  const int rc = check_launch("tedq_sv_expval_factored(partial)");
+  if (rc) return rc;
+  sum_partials(partial, batch * count, nchunk, 1, out, st);
+  return check_launch("tedq_sv_expval_factored(sum)");
 }
 
 extern "C" int tedq_sv_expval_factored(const void* state, int64_t batch, int n_qubits, int q, const int* bits,
@@ -666,15 +810,53 @@ extern "C" int tedq_sv_expval_factored(const void* state, int64_t batch, int n_q
     set_error("tedq_sv_expval_factored: bad arguments (q=%d)", q);
     return kBadArgument;
   }
-  const int64_t ngroups = 1ll << (n_qubits - q);
-  const int64_t nchunk = tedq_sv_reduce_chunks(n_qubits);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_expval_factored, dim3((unsigned)nchunk, (unsigned)batch), dim3(kRedThreads), 0, st,
-                     static_cast<const float2*>(state), n_qubits, o, partial, ngroups, nchunk);
-  int rc = check_launch("tedq_sv_expval_factored(partial)");
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_sum_partials<double>, dim3(nblocks(batch, 128)), dim3(128), 0, st, partial, batch, nchunk, 1, out);
-  return check_launch("tedq_sv_expval_factored(sum)");
+  return launch_expval_factored(state, batch, n_qubits, q, nullptr, o, 1, tedq_sv_reduce_chunks(n_qubits), partial, out,
+                                static_cast<hipStream_t>(stream));
+}
+
+// Records of the batched form: sizeof(FactorObs) bytes each, filled by tedq_sv_factored_record on the host
+// and copied to the device by the caller.
+extern "C" int64_t tedq_sv_factored_record_bytes(void) { return (int64_t)sizeof(FactorObs); }
+
+extern "C" int tedq_sv_factored_record(void* record, int n_qubits, int q, const int* bits, const float* factors,
+                                       uint64_t zmask) {
+  FactorObs o = {};
+  if (record == nullptr || n_qubits < 1 || n_qubits > 40 || q > n_qubits ||
+      make_factor_obs(&o, n_qubits, q, bits, factors, zmask) != kOk) {
+    set_error("tedq_sv_factored_record: bad arguments (q=%d)", q);
+    return kBadArgument;
+  }
+  memcpy(record, &o, sizeof(o));
+  return kOk;
+}
+
+extern "C" int64_t tedq_sv_factored_chunks(int n_qubits, int q) {
+  if (n_qubits < 1 || n_qubits > 40 || q < 0 || q > 4 || q > n_qubits) return -1;
+  const int lg = n_qubits - q - 11;
+  return lg <= 0 ? 1 : (lg > 10 ? 1024 : 1ll << lg);
+}
+
+static int factored_records_ok(const void* records, int count, int n_qubits, int q) {
+  const FactorObs* o = static_cast<const FactorObs*>(records);
+  for (int i = 0; i < count; ++i) {
+    if (o[i].q != q) return 0;
+    for (int j = 0; j < q; ++j)
+      if (o[i].bits[j] < 0 || o[i].bits[j] >= n_qubits || (j > 0 && o[i].sorted[j] < o[i].sorted[j - 1])) return 0;
+  }
+  return 1;
+}
+
+extern "C" int tedq_sv_expval_factored_batch(const void* state, int64_t batch, int n_qubits, int q,
+                                             const void* records, const void* records_dev, int count,
+                                             double* partial, double* out, void* stream) {
+  if (state == nullptr || records == nullptr || records_dev == nullptr || partial == nullptr || out == nullptr ||
+      batch <= 0 || batch > 65535 || count <= 0 || count > 65535 || n_qubits < 1 || n_qubits > 40 || q < 0 || q > 4 ||
+      q > n_qubits || !factored_records_ok(records, count, n_qubits, q)) {
+    set_error("tedq_sv_expval_factored_batch: bad arguments (q=%d count=%d)", q, count);
+    return kBadArgument;
+  }
+  return launch_expval_factored(state, batch, n_qubits, q, static_cast<const FactorObs*>(records_dev), FactorObs{}, count,
+                                tedq_sv_factored_chunks(n_qubits, q), partial, out, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tedq_sv_lambda_factored(const void* psi, void* lam, int64_t batch, int n_qubits, int q,
@@ -687,10 +869,29 @@ extern "C" int tedq_sv_lambda_factored(const void* psi, void* lam, int64_t batch
     return kBadArgument;
   }
   const int64_t ngroups = 1ll << (n_qubits - q);
-  hipLaunchKernelGGL(k_lambda_factored, dim3(nblocks(batch * ngroups, 256)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), static_cast<const float2*>(psi), static_cast<float2*>(lam),
-                     n_qubits, o, ngroups, coef, batch);
+#define TEDQ_LAUNCH(Q)                                                                                       \
+  hipLaunchKernelGGL(k_lambda_factored<Q>, dim3(nblocks(batch * ngroups, 256)), dim3(256), 0,                \
+                     static_cast<hipStream_t>(stream), static_cast<const float2*>(psi), static_cast<float2*>(lam), \
+                     n_qubits, o, ngroups, coef, batch)
+  TEDQ_FACTORED_CASES(TEDQ_LAUNCH)
+#undef TEDQ_LAUNCH
   return check_launch("tedq_sv_lambda_factored");
+}
+
+extern "C" int tedq_sv_lambda_factored_batch(const void* psi, void* lam, int64_t batch, int n_qubits,
+                                             const void* records, const void* records_dev, int count,
+                                             const double* coef, void* stream) {
+  if (psi == nullptr || lam == nullptr || psi == lam || records == nullptr || records_dev == nullptr ||
+      coef == nullptr || batch <= 0 || count <= 0 || n_qubits < 1 || n_qubits > 40 ||
+      !factored_records_ok(records, count, n_qubits, 1)) {
+    set_error("tedq_sv_lambda_factored_batch: bad arguments (count=%d)", count);
+    return kBadArgument;
+  }
+  const int64_t total = batch << n_qubits;
+  hipLaunchKernelGGL(k_lambda_factored1, dim3(nblocks(total, 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const float2*>(psi), static_cast<float2*>(lam), n_qubits,
+                     static_cast<const FactorObs*>(records_dev), count, coef, total);
+  return check_launch("tedq_sv_lambda_factored_batch");
 }
 
 static int make_bitlist(BitList* bl, int n, int k, const int* bits, const char* what) {
@@ -748,8 +949,7 @@ extern "C" int tedq_sv_probs(const void* state, int64_t batch, int n_qubits, int
                      static_cast<const float2*>(state), n_qubits, bl, rest_mask_of(bl, n_qubits), partial, nrc);
   rc = check_launch("tedq_sv_probs(partial)");
   if (rc) return rc;
-  hipLaunchKernelGGL(k_sum_partials<float>, dim3(nblocks(batch << k, 128)), dim3(128), 0, st, partial, batch, nrc,
-                     1 << k, out);
+  sum_partials(partial, batch, nrc, 1ll << k, out, st);
   return check_launch("tedq_sv_probs(sum)");
 }
 
@@ -803,8 +1003,7 @@ extern "C" int tedq_sum_partials(const double* partial, int64_t batch, int64_t n
     set_error("tedq_sum_partials: bad arguments");
     return kBadArgument;
   }
-  hipLaunchKernelGGL(k_sum_partials<double>, dim3(nblocks(batch * M, 128)), dim3(128), 0, static_cast<hipStream_t>(stream),
-                     partial, batch, nchunk, M, out);
+  sum_partials(partial, batch, nchunk, M, out, static_cast<hipStream_t>(stream));
   return check_launch("tedq_sum_partials");
 }
 

@@ -577,6 +577,15 @@ class SVExecutor:
                 raise hip.EngineError(f"state norm check failed: max |<psi|psi> - 1| = {dev_max:.3e} over "
                                       f"{B} rows exceeds {self.norm_tol:.1e}")
         outs = []
+        factored = {}
+        for q, (specs, recs, drecs) in self._factored_records(dev).items():
+            nf = len(specs)
+            partial = torch.empty((B, nf, hip.load().tedq_sv_factored_chunks(self.n, q)), dtype=torch.float64,
+                                  device=dev)
+            fout = torch.empty((B, nf), dtype=torch.float64, device=dev)
+            hip.call("tedq_sv_expval_factored_batch", hip.ptr(psi), B, self.n, q, _hptr(recs), hip.ptr(drecs), nf,
+                     hip.ptr(partial), hip.ptr(fout), st)
+            factored.update({id(spec): fout[:, i] for i, spec in enumerate(specs)})
         for spec in self.specs:
             if spec.kind == "zexp":
                 outs.append(zout[:, spec.zindex])
@@ -590,12 +599,7 @@ class SVExecutor:
                          hip.ptr(vals), st)
                 outs.append(vals @ torch.tensor(spec.bcoefs, dtype=torch.float64, device=dev))
             elif spec.kind == "fexp":
-                bits, fac = _factored_args(spec, dev)
-                partial = torch.empty((B, nchunk), dtype=torch.float64, device=dev)
-                out = torch.empty((B,), dtype=torch.float64, device=dev)
-                hip.call("tedq_sv_expval_factored", hip.ptr(psi), B, self.n, len(spec.fbits), _hptr(bits),
-                         _hptr(fac), spec.zmask, hip.ptr(partial), hip.ptr(out), st)
-                outs.append(out)
+                outs.append(factored[id(spec)])
             elif spec.kind == "probs":
                 k = len(spec.pbits) if spec.pbits else self.n
                 out = torch.empty((B, 2 ** k), dtype=torch.float32, device=dev)
@@ -611,6 +615,25 @@ class SVExecutor:
             else:
                 outs.append(psi.view((B,) + spec.shape))
         return outs
+
+    def _factored_records(self, device):
+        """{factor count: (specs, host records, device copy)} of the factored observables."""
+        key = ("factored", device.type, device.index)
+        if key not in self._dev:
+            groups = {}
+            for spec in self.specs:
+                if spec.kind == "fexp" and spec.basis is None:
+                    groups.setdefault(len(spec.fbits), []).append(spec)
+            size = hip.load().tedq_sv_factored_record_bytes() if groups else 0
+            out = {}
+            for q, specs in groups.items():
+                recs = np.zeros((len(specs), size), dtype=np.uint8)
+                for rec, spec in zip(recs, specs):
+                    bits, fac = _factored_args(spec, device)
+                    hip.call("tedq_sv_factored_record", _hptr(rec), self.n, q, _hptr(bits), _hptr(fac), spec.zmask)
+                out[q] = (specs, recs, torch.from_numpy(recs.copy()).to(device))
+            self._dev[key] = out
+        return self._dev[key]
 
     def _basis_program(self, spec, inverse):
         """Pass program applying V_i^dagger (inverse) or V_i to every factor bit of a basis spec."""
@@ -708,8 +731,18 @@ class SVExecutor:
             coef = cols[m].contiguous()
             hip.call("tedq_sv_lambda_factored", hip.ptr(psi), hip.ptr(lam), B, self.n, 0, None, None,
                      self.zmasks[m], hip.ptr(coef), st)
+        # one-factor observables, when all of them have a gradient: one launch
+        up = {id(spec): g for spec, g in zip(self.specs, grads)}
+        one, recs, drecs = self._factored_records(dev).get(1, ((), None, None))
+        if one and all(up[id(spec)] is not None for spec in one):
+            coef = torch.stack([up[id(spec)].to(torch.float64).reshape(B) for spec in one], 1).contiguous()
+            hip.call("tedq_sv_lambda_factored_batch", hip.ptr(psi), hip.ptr(lam), B, self.n, _hptr(recs),
+                     hip.ptr(drecs), len(one), hip.ptr(coef), st)
+        else:
+            one = ()
+        done = {id(spec) for spec in one}
         for spec, g in zip(self.specs, grads):
-            if g is None or spec.kind == "zexp":
+            if g is None or spec.kind == "zexp" or id(spec) in done:
                 continue
             if spec.kind == "fexp" and spec.basis is not None:
                 # lam += g O psi with O = (x V) [sum_S c_S Z_S] (x V^dagger)
