@@ -30,7 +30,7 @@ namespace {
 constexpr int kTileMax = 12, kTileMin = 9, kOuterMax = 20;
 constexpr int kRunOps = 32, kRunCoef = 512;
 constexpr int kOpWords = 52, kPassWords = 128, kFactors = 4;
-constexpr int kBwdThreads = 512;
+constexpr int kBwdLog = 9, kBwdThreads = 1 << kBwdLog;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -60,23 +60,27 @@ __device__ __forceinline__ uint32_t insert0(uint32_t r, int p) {
   return ((r >> p) << (p + 1)) | (r & ((1u << p) - 1u));
 }
 
-// row r of an op of arity A: the tile element with the op's slots clear
+// LDS byte of row r of an op of arity A: the tile element with the op's slots
+// clear.  Linear (XOR) in the bits of r: the part of a thread's own bits is
+// formed once per op, the rest is uniform and left to the scalar unit.
 template <int A>
-__device__ __forceinline__ uint32_t row_word(uint32_t r, const int* s) {
+__device__ __forceinline__ uint32_t row_byte(uint32_t r, const int* s) {
   uint32_t a = insert0(insert0(r, s[0]), s[1]);
   if (A == 3) a = insert0(a, s[2]);
-  return sw(a);
+  return sw(a) << 3;
 }
 
+// LDS byte offset of element k of a row
 template <int A>
-__device__ __forceinline__ void slot_words(const int* s, uint32_t* o) {
+__device__ __forceinline__ uint32_t slot_byte(uint32_t k, const int* s) {
+  uint32_t a = 0;
 #pragma unroll
-  for (int k = 0; k < (1 << A); ++k) {
-    uint32_t a = 0;
-#pragma unroll
-    for (int j = 0; j < A; ++j) a |= ((k >> j) & 1u) << s[j];
-    o[k] = sw(a);
-  }
+  for (int j = 0; j < A; ++j) a |= ((k >> j) & 1u) << s[j];
+  return sw(a) << 3;
+}
+
+__device__ __forceinline__ float2& at(float2* base, uint32_t byte) {
+  return *reinterpret_cast<float2*>(reinterpret_cast<char*>(base) + byte);
 }
 
 __device__ __forceinline__ f32x4 mm(float a, float b, f32x4 c) {
@@ -87,8 +91,9 @@ __device__ __forceinline__ f32x4 mm(float a, float b, f32x4 c) {
 template <int A>
 __device__ __forceinline__ void apply_op(float2* tile, const float2* m, const int* s, int n_local, int threads) {
   constexpr int D = 1 << A, Q = D / 4;
-  const int t = threadIdx.x;
-  float ar[Q][D], ai[Q][D];
+  const int t = threadIdx.x, rows = 1 << (n_local - A);
+  if (t >= rows) return;  // whole waves
+  float ar[Q][D], ai[Q][D], an[Q][D];
 #pragma unroll
   for (int q = 0; q < Q; ++q)
 #pragma unroll
@@ -96,28 +101,27 @@ __device__ __forceinline__ void apply_op(float2* tile, const float2* m, const in
       const float2 v = m[(4 * q + (t & 3)) * D + k];
       ar[q][k] = v.x;
       ai[q][k] = v.y;
+      an[q][k] = -v.y;
     }
-  uint32_t o[D];
-  slot_words<A>(s, o);
-  const int rows = 1 << (n_local - A);
+  const uint32_t w0 = row_byte<A>(t, s);
 #pragma unroll 2
-  for (int r = t; r < rows; r += threads) {
-    const uint32_t w = row_word<A>(r, s);
+  for (int r = 0; r < rows; r += threads) {
+    const uint32_t w = w0 ^ row_byte<A>(r, s);
     float2 x[D];
 #pragma unroll
-    for (int k = 0; k < D; ++k) x[k] = tile[w ^ o[k]];
+    for (int k = 0; k < D; ++k) x[k] = at(tile, w ^ slot_byte<A>(k, s));
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       f32x4 re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < D; ++k) {
-        re = mm(ai[q][k], -x[k].y, re);
+        re = mm(an[q][k], x[k].y, re);
         im = mm(ai[q][k], x[k].x, im);
         re = mm(ar[q][k], x[k].x, re);
         im = mm(ar[q][k], x[k].y, im);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) tile[w ^ o[4 * q + i]] = make_float2(re[i], im[i]);
+      for (int i = 0; i < 4; ++i) at(tile, w ^ slot_byte<A>(4 * q + i, s)) = make_float2(re[i], im[i]);
     }
   }
 }
@@ -162,7 +166,8 @@ __global__ void __launch_bounds__(64) k_tn_run_coefs(TNRunBases bases, const int
 // One forward pass: workgroup (g, b) owns tile g of batch element b.
 // 256 threads and 32 KB of LDS at 2^12 elements: five workgroups per CU, whose
 // loads, matrices and stores overlap.  Measured on 2^25 elements with 8
-// matrices per pass: 198 us a pass, against 8 x 92 us step by step.
+// matrices per pass: 189 us a pass (94 us + 15 us per
+// matrix), against 8 x 92 us step by step.
 template <bool A3>
 __global__ void __launch_bounds__(256) k_tn_run_pass(const float2* __restrict__ X, int64_t x_bs,
                                                      float2* __restrict__ C, int64_t c_bs,
@@ -257,58 +262,57 @@ __device__ __forceinline__ void undo_op(float2* xt, float2* et, const float2* m,
   constexpr int D = 1 << A, Q = D / 4;
   const int t = threadIdx.x, lane = t & 63, i4 = lane & 3;
   const int rows = 1 << (n_local - A);
-  if ((t & ~63) >= rows) return;  // whole waves
-  uint32_t o[D];
-  slot_words<A>(s, o);
-  uint32_t oi[Q];
-#pragma unroll
-  for (int q = 0; q < Q; ++q) {
-    uint32_t a = 0;
-#pragma unroll
-    for (int j = 0; j < A; ++j) a |= (((4 * q + i4) >> j) & 1u) << s[j];
-    oi[q] = sw(a);
-  }
-  f32x4 gr[Q][Q], gi[Q][Q];
+  if (t >= rows) return;  // whole waves
+  const uint32_t w0 = row_byte<A>(t, s);
+  const uint32_t wt0 = row_byte<A>((t & ~63) | (lane >> 2), s) ^ slot_byte<A>(i4, s);
+  f32x4 gr[Q][Q], gn[Q][Q], gi[Q][Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q)
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
-      gr[q][k] = {0.f, 0.f, 0.f, 0.f};
-      gi[q][k] = {0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < Q; ++k) gr[q][k] = gn[q][k] = gi[q][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // arity 2 keeps its column of the matrix in registers, arity 3 reads it again
+  float mr[A == 2 ? D : 1], mi[A == 2 ? D : 1], mn[A == 2 ? D : 1];
+  if (A == 2)
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      const float2 v = m[k * D + i4];
+      mr[A == 2 ? k : 0] = v.x;
+      mi[A == 2 ? k : 0] = v.y;
+      mn[A == 2 ? k : 0] = -v.y;
     }
-  for (int r = t; r < rows; r += kBwdThreads) {
-    const uint32_t w = row_word<A>(r, s);
+  for (int r = 0; r < rows; r += kBwdThreads) {
+    const uint32_t wr = row_byte<A>(r, s), w = w0 ^ wr;
     float2 x[D], e[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-      x[k] = xt[w ^ o[k]];
-      e[k] = et[w ^ o[k]];
+      x[k] = at(xt, w ^ slot_byte<A>(k, s));
+      e[k] = at(et, w ^ slot_byte<A>(k, s));
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       f32x4 re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < D; ++k) {
-        const float2 v = m[k * D + 4 * q + i4];
+        const float2 v = A == 2 ? make_float2(mr[A == 2 ? k : 0], mi[A == 2 ? k : 0]) : m[k * D + 4 * q + i4];
+        const float vn = A == 2 ? mn[A == 2 ? k : 0] : -v.y;
         re = mm(v.y, x[k].y, re);
-        im = mm(v.y, -x[k].x, im);
+        im = mm(vn, x[k].x, im);
         re = mm(v.x, x[k].x, re);
         im = mm(v.x, x[k].y, im);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) xt[w ^ o[4 * q + i]] = make_float2(re[i], im[i]);
+      for (int i = 0; i < 4; ++i) at(xt, w ^ slot_byte<A>(4 * q + i, s)) = make_float2(re[i], im[i]);
     }
     __builtin_amdgcn_wave_barrier();
     asm volatile("" ::: "memory");
-    const uint32_t r0 = (uint32_t)(r & ~63) + (lane >> 2);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const uint32_t wt = row_word<A>(r0 + 16 * u, s);
+      const uint32_t wt = wt0 ^ (wr ^ row_byte<A>(16 * u, s));
       float2 xv[Q], ev[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        xv[q] = xt[wt ^ oi[q]];
-        ev[q] = et[wt ^ oi[q]];
+        xv[q] = at(xt, wt ^ slot_byte<A>(4 * q, s));
+        ev[q] = at(et, wt ^ slot_byte<A>(4 * q, s));
       }
 #pragma unroll
       for (int q = 0; q < Q; ++q)
@@ -316,7 +320,7 @@ __device__ __forceinline__ void undo_op(float2* xt, float2* et, const float2* m,
         for (int k = 0; k < Q; ++k) {
           gr[q][k] = mm(ev[q].x, xv[k].x, gr[q][k]);
           gi[q][k] = mm(ev[q].x, xv[k].y, gi[q][k]);
-          gr[q][k] = mm(-ev[q].y, xv[k].y, gr[q][k]);
+          gn[q][k] = mm(ev[q].y, xv[k].y, gn[q][k]);
           gi[q][k] = mm(ev[q].y, xv[k].x, gi[q][k]);
         }
     }
@@ -327,14 +331,15 @@ __device__ __forceinline__ void undo_op(float2* xt, float2* et, const float2* m,
       f32x4 re = {0.f, 0.f, 0.f, 0.f}, im = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < D; ++k) {
-        const float2 v = m[k * D + 4 * q + i4];
-        re = mm(-v.y, e[k].y, re);
+        const float2 v = A == 2 ? make_float2(mr[A == 2 ? k : 0], mi[A == 2 ? k : 0]) : m[k * D + 4 * q + i4];
+        const float vn = A == 2 ? mn[A == 2 ? k : 0] : -v.y;
+        re = mm(vn, e[k].y, re);
         im = mm(v.y, e[k].x, im);
         re = mm(v.x, e[k].x, re);
         im = mm(v.x, e[k].y, im);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) et[w ^ o[4 * q + i]] = make_float2(re[i], im[i]);
+      for (int i = 0; i < 4; ++i) at(et, w ^ slot_byte<A>(4 * q + i, s)) = make_float2(re[i], im[i]);
     }
   }
   float* rw = red + (t >> 6) * (2 * D * D);
@@ -342,7 +347,7 @@ __device__ __forceinline__ void undo_op(float2* xt, float2* et, const float2* m,
   for (int q = 0; q < Q; ++q)
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-      const float v = block_sum(gr[q][k], gi[q][k], lane);
+      const float v = block_sum(gr[q][k] - gn[q][k], gi[q][k], lane);
       const int row = 4 * q + ((lane >> 3) & 3), col = 4 * k + i4;
       if ((lane & 4) == 0) rw[2 * (row * D + col) + (lane >> 5)] = v;
     }
@@ -355,7 +360,8 @@ __device__ __forceinline__ void undo_op(float2* xt, float2* et, const float2* m,
 // partial sums written are per workgroup, not per tile.  EX may be EC when the
 // pass keeps the layout: a tile is read whole before it is written.
 // 512 threads, two tiles of 32 KB: two workgroups, 16 waves per CU.  Measured
-// on 2^25 elements with 8 matrices per pass: 535 us, against 8 x 152 us.
+// on 2^25 elements with 8 matrices per pass: 503 us (130 us + 52 us per matrix),
+// against 8 x 152 us.
 template <bool A3>
 __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __restrict__ C, int64_t c_bs,
                                                             const float2* EC, int64_t ec_bs, float2* EX,
@@ -363,11 +369,12 @@ __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __rest
                                                             int64_t coef_bs, const int32_t* __restrict__ ops,
                                                             float* __restrict__ part, TNRunPlan P) {
   extern __shared__ float2 lds[];
+  constexpr int kPer = 1 << (kTileMax - kBwdLog);
   constexpr int kRed = (kBwdThreads / 64) * (A3 ? 128 : 32);
   const int t = threadIdx.x, N = 1 << P.n_local;
   float2* xt = lds;
-  float2* et = lds + N;
-  float2* m = lds + 2 * N;
+  float2* et = lds + (1 << kTileMax);  // a constant distance: one address serves both
+  float2* m = lds + (2 << kTileMax);
   float* acc = reinterpret_cast<float*>(m + P.coef);
   float* red = acc + 2 * P.coef;
   const int64_t b = blockIdx.y;
@@ -376,7 +383,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __rest
   for (int e = t; e < 2 * P.coef; e += kBwdThreads) acc[e] = 0.f;
   uint32_t lo_in = 0, lo_out = 0, ls = 0;
 #pragma unroll
-  for (int i = 0; i < 9; ++i) {
+  for (int i = 0; i < kBwdLog; ++i) {
     lo_in |= ((t >> i) & 1u) << P.in_bit[i];
     lo_out |= ((t >> i) & 1u) << P.out_bit[i];
     ls |= ((t >> i) & 1u) << P.out_slot[i];
@@ -386,22 +393,22 @@ __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __rest
     const uint32_t oo = lo_out | outer_offset(g, P.n_outer, P.outer_out);
     const float2* c = C + b * c_bs + oo;
     const float2* ec = EC + b * ec_bs + oo;
-    float2 vx[8], ve[8];
+    float2 vx[kPer], ve[kPer];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < kPer; ++j) {
       uint32_t hi = 0;
 #pragma unroll
-      for (int i = 0; i < 3; ++i) hi |= ((j >> i) & 1u) << P.out_bit[9 + i];
+      for (int i = 0; i < kTileMax - kBwdLog; ++i) hi |= ((j >> i) & 1u) << P.out_bit[kBwdLog + i];
       if (j * kBwdThreads < N) {
         vx[j] = c[hi];
         ve[j] = ec[hi];
       }
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < kPer; ++j) {
       uint32_t hs = 0;
 #pragma unroll
-      for (int i = 0; i < 3; ++i) hs |= ((j >> i) & 1u) << P.out_slot[9 + i];
+      for (int i = 0; i < kTileMax - kBwdLog; ++i) hs |= ((j >> i) & 1u) << P.out_slot[kBwdLog + i];
       if (j * kBwdThreads < N) {
         xt[sw(hs | ls)] = vx[j];
         et[sw(hs | ls)] = ve[j];
@@ -429,10 +436,10 @@ __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __rest
     }
     float2* ex = EX + b * ex_bs + (lo_in | outer_offset(g, P.n_outer, P.outer_in));
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < kPer; ++j) {
       uint32_t hi = 0;
 #pragma unroll
-      for (int i = 0; i < 3; ++i) hi |= ((j >> i) & 1u) << P.in_bit[9 + i];
+      for (int i = 0; i < kTileMax - kBwdLog; ++i) hi |= ((j >> i) & 1u) << P.in_bit[kBwdLog + i];
       if (j * kBwdThreads < N) ex[hi] = et[sw(j * kBwdThreads + t)];
     }
     __syncthreads();
@@ -444,18 +451,22 @@ __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __rest
 // Environment of an op's gate: the workgroups' sums of its matrix entries,
 // written to the gate tensor's own address order (an op on one address bit
 // carries a spectator bit, which is summed here).
-__global__ void __launch_bounds__(256) k_tn_run_env(const float* __restrict__ part, int n_wg, int coef,
-                                                    const int32_t* __restrict__ ops, float2* env0, int64_t bs0,
-                                                    float2* env1, int64_t bs1) {
-  __shared__ double sum[256];
+// 1024 threads: the workgroups' rows are 128 B apart reads of one matrix, a
+// chain of loads per thread (39 us per pass with 256 threads and no unrolling).
+__global__ void __launch_bounds__(1024) k_tn_run_env(const float* __restrict__ part, int n_wg, int coef,
+                                                     const int32_t* __restrict__ ops, float2* env0, int64_t bs0,
+                                                     float2* env1, int64_t bs1) {
+  __shared__ double sum[1024];
   __shared__ float2 val[64];
   const int32_t* w = ops + (int64_t)blockIdx.x * kOpWords;
   if (w[W_EBASE] < 0) return;
   const int64_t b = blockIdx.y;
   const int t = threadIdx.x, a = w[W_ARITY], size = 2 << (2 * a), off = 2 * (w[W_COEF] - ops[W_COEF]);
-  const int v = t & (size - 1), step = 256 / size;
+  const int step = 1024 / size;
+  const float* p = part + b * n_wg * (int64_t)(2 * coef) + off + (t & (size - 1));
   double s = 0.0;
-  for (int g = t / size; g < n_wg; g += step) s += part[(b * n_wg + g) * (int64_t)(2 * coef) + off + v];
+#pragma unroll 8
+  for (int g = t / size; g < n_wg; g += step) s += p[g * (int64_t)(2 * coef)];
   sum[t] = s;
   __syncthreads();
   if (t < size) {
@@ -663,7 +674,7 @@ extern "C" int tedq_tn_run_backward(const void* c, int64_t c_bs, const void* ec,
               (long long)workspace_bytes);
     return kBadArgument;
   }
-  const size_t lds = sizeof(float2) * (2 * (size_t)(1 << P.n_local) + P.coef) + sizeof(float) * 2 * P.coef +
+  const size_t lds = sizeof(float2) * ((size_t)(2 << kTileMax) + P.coef) + sizeof(float) * 2 * P.coef +
                      sizeof(float) * 2 * (kBwdThreads / 64) * (a3 ? 128 : 32);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)groups, (unsigned)batch);
@@ -683,7 +694,7 @@ extern "C" int tedq_tn_run_backward(const void* c, int64_t c_bs, const void* ec,
                        static_cast<const float2*>(coef), coef_bs, ops_dev, static_cast<float*>(workspace), P);
   const int rc = check_launch("tedq_tn_run_backward");
   if (rc != kOk) return rc;
-  hipLaunchKernelGGL(k_tn_run_env, dim3((unsigned)P.n_ops, (unsigned)batch), dim3(256), 0, st,
+  hipLaunchKernelGGL(k_tn_run_env, dim3((unsigned)P.n_ops, (unsigned)batch), dim3(1024), 0, st,
                      static_cast<const float*>(workspace), groups, P.coef, ops_dev, static_cast<float2*>(env0), bs0,
                      static_cast<float2*>(env1), bs1);
   return check_launch("tedq_tn_run_backward(env)");
