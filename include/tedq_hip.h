@@ -259,6 +259,12 @@ int tedq_tn_contract(const void* a, int64_t a_bstride, const void* b, int64_t b_
 int tedq_tn_contract_small_batch(const void* const* bases, const int64_t* strides, const int64_t* lens,
                                  const int64_t* records, const int64_t* records_dev, int n_records, int64_t batch,
                                  const int32_t* descs, const int32_t* descs_dev, int n_descs, void* stream);
+/* The environment steps of small steps, one tree level in one launch: as
+ * above with five arenas, at most 2^12 summed terms per output, and word 7 of a
+ * record naming the arena of its result. */
+int tedq_tn_small_environments(const void* const* bases, const int64_t* strides, const int64_t* lens,
+                               const int64_t* records, const int64_t* records_dev, int n_records, int64_t batch,
+                               const int32_t* descs, const int32_t* descs_dev, int n_descs, void* stream);
 /* Both environments of a gate step in one pass.  desc: the forward step C = A B
  * (host + device copies as in tedq_tn_contract) with one operand X large (at
  * least 2^10 rows) and the other G gate-sized (at most two summed and two new

@@ -36,7 +36,7 @@
 //     next k chunk, for steps whose m and n are both at least 128 wide (both
 //     GEMM kernels split long sums over workgroups when tiles are few);
 //   * k_tn_small_multi (tedq_tn_contract_small_batch): every small step of
-//     one level of the contraction tree in one launch;
+//     one level of the contraction tree in one launch, forward or backward;
 //   * k_tn_gate_bwd (tedq_tn_gate_backward): both environments of a
 //     k_tn_gate step from one read of the result's environment.
 // Arithmetic is complex64 with fp32 accumulation, like the reference's
@@ -439,23 +439,26 @@ static TNPermPlan perm_plan(const TNDesc& d, int a_tensor) {
 }
 
 // Many small steps in one launch (the gate-merging steps of a contraction
-// path: every operand a leaf or the result of another small step).  Workgroup
-// (r, b) runs step r of the list for batch element b: outputs in C's address
-// order over the threads, each summed over all 2^nK terms.  A record is eight
-// int64: descriptor row, A base id, A element offset, B base id, B offset,
-// C offset (in base 2), output count, reserved; a base id selects one of the
-// three (pointer, batch stride) pairs passed by value.
+// path: every operand a leaf or the result of another small step; backward:
+// the environment steps of those).  Workgroup (r, b) runs step r of the list
+// for batch element b: a group of 2^lpo lanes per output, adjacent in k, where
+// the outputs alone would leave threads idle (a gate's environment has 16
+// outputs summed over up to 2^10 terms).  A record is eight int64: descriptor
+// row, A base id, A element offset, B base id, B offset, C offset, output
+// count, C base id; a base id selects one of the (pointer, batch stride) pairs
+// passed by value.  One launch per tree level: a 5x5 lattice's backward had
+// 1172 launches of 4 us (a launch's own latency) for these steps, now 25 of 13 us.
+constexpr int kSmallBases = 5;
 struct TNBases {
-  const float2* p[3];
-  int64_t stride[3];
+  float2* p[kSmallBases];
+  int64_t stride[kSmallBases];
 };
 
-__global__ void __launch_bounds__(256) k_tn_small_multi(TNBases bases, float2* __restrict__ out_base,
-                                                        const int64_t* __restrict__ recs,
-                                                        const int32_t* __restrict__ descs) {
+__global__ void __launch_bounds__(256) k_tn_small_multi(TNBases bases, const int64_t* __restrict__ recs,
+                                                        const int32_t* __restrict__ descs, int c_base) {
   __shared__ TNShared d;
   __shared__ signed char mapA[32], mapB[32];
-  __shared__ uint32_t tka[64], tkb[64];
+  __shared__ uint32_t tka[1 << kTabBits], tkb[1 << kTabBits];
   const int64_t* rec = recs + 8 * (int64_t)blockIdx.x;
   const int row = (int)rec[0];
   load_desc(d, descs + (int64_t)row * (4 + 9 * 32));
@@ -463,28 +466,44 @@ __global__ void __launch_bounds__(256) k_tn_small_multi(TNBases bases, float2* _
   const int nH = d.nb[0], nM = d.nb[1], nN = d.nb[2], nK = d.nb[3];
   const int rc = nH + nM + nN;
   const int t = threadIdx.x;
-  if (t < (1 << nK)) {
-    tka[t] = scat(d, AK, nK, t);
-    tkb[t] = scat(d, BK, nK, t);
+  const int kt = nK < kTabBits ? nK : kTabBits;
+  for (int k = t; k < (1 << kt); k += 256) {
+    tka[k] = scat(d, AK, kt, k);
+    tkb[k] = scat(d, BK, kt, k);
   }
   __syncthreads();
   const int64_t b = blockIdx.y;
-  const int ia = (int)rec[1], ib = (int)rec[3];
+  const int ia = (int)rec[1], ib = (int)rec[3], ic = c_base >= 0 ? c_base : (int)rec[7];
   const float2* a = bases.p[ia] + b * bases.stride[ia] + rec[2];
   const float2* bp = bases.p[ib] + b * bases.stride[ib] + rec[4];
-  float2* c = out_base + b * bases.stride[2] + rec[5];
+  float2* c = bases.p[ic] + b * bases.stride[ic] + rec[5];
   const int n_out = (int)rec[6];
-  const int kc = 1 << nK;
-  for (int o = t; o < n_out; o += 256) {
+  int lpo = 0;
+  while (lpo < 6 && lpo < nK && (n_out << lpo) < 256) ++lpo;
+  // whole groups of lanes leave the loop together, so the shuffles see every lane of a group
+  for (int i = t; i < (n_out << lpo); i += 256) {
+    const int o = i >> lpo;
     const uint32_t oa = via_map(mapA, rc, (uint32_t)o), ob = via_map(mapB, rc, (uint32_t)o);
     float2 acc = make_float2(0.f, 0.f);
-    for (int k = 0; k < kc; ++k) {
-      const float2 x = a[oa | tka[k]];
-      const float2 y = bp[ob | tkb[k]];
-      acc.x = fmaf(x.x, y.x, fmaf(-x.y, y.y, acc.x));
-      acc.y = fmaf(x.x, y.y, fmaf(x.y, y.x, acc.y));
+    for (int kh = 0; kh < (1 << (nK - kt)); ++kh) {
+      uint32_t ha = oa, hb = ob;
+      for (int j = kt; j < nK; ++j) {
+        const uint32_t bit = ((uint32_t)kh >> (j - kt)) & 1u;
+        ha |= bit << d.pos[AK][j];
+        hb |= bit << d.pos[BK][j];
+      }
+      for (int k = i & ((1 << lpo) - 1); k < (1 << kt); k += 1 << lpo) {
+        const float2 x = a[ha | tka[k]];
+        const float2 y = bp[hb | tkb[k]];
+        acc.x = fmaf(x.x, y.x, fmaf(-x.y, y.y, acc.x));
+        acc.y = fmaf(x.x, y.y, fmaf(x.y, y.x, acc.y));
+      }
     }
-    c[o] = acc;
+    for (int h = (1 << lpo) >> 1; h > 0; h >>= 1) {
+      acc.x += __shfl_xor(acc.x, h, 64);
+      acc.y += __shfl_xor(acc.y, h, 64);
+    }
+    if ((i & ((1 << lpo) - 1)) == 0) c[o] = acc;
   }
 }
 
@@ -1301,52 +1320,71 @@ extern "C" int tedq_tn_contract(const void* a, int64_t a_bstride, const void* b,
 }
 
 // Small steps of one tree level in one launch (see k_tn_small_multi).  bases /
-// strides / lens: three operand arenas (device pointers, per-batch strides in
-// elements, elements valid per batch row); base 2 is also where every result
-// goes.  records / records_dev: n_records records of 8 int64, host and device
-// copies; descs / descs_dev: the descriptor table (n_descs rows), host and
-// device copies.  Each step must have rank <= 12 operands and results, at most
-// 2^6 summed terms, and fit its arenas (all checked on the host).
-extern "C" int tedq_tn_contract_small_batch(const void* const* bases, const int64_t* strides, const int64_t* lens,
-                                            const int64_t* records, const int64_t* records_dev, int n_records,
-                                            int64_t batch, const int32_t* descs, const int32_t* descs_dev,
-                                            int n_descs, void* stream) {
+// strides / lens: operand arenas (device pointers, per-batch strides in
+// elements, elements valid per batch row); records / records_dev: n_records
+// records of 8 int64, host and device copies; descs / descs_dev: the descriptor
+// table (n_descs rows), host and device copies.  Each step must have rank <= 12
+// operands and results, at most 2^max_k summed terms, and fit its arenas (all
+// checked on the host).  c_base >= 0: every result goes to that arena.
+static int launch_small(const char* what, const void* const* bases, const int64_t* strides, const int64_t* lens,
+                        int n_bases, const int64_t* records, const int64_t* records_dev, int n_records, int64_t batch,
+                        const int32_t* descs, const int32_t* descs_dev, int n_descs, int c_base, int max_k,
+                        void* stream) {
   if (bases == nullptr || strides == nullptr || lens == nullptr || records == nullptr || records_dev == nullptr ||
       descs == nullptr || descs_dev == nullptr || n_records < 0 || n_descs <= 0 || batch <= 0 || batch > 65535) {
-    set_error("tedq_tn_contract_small_batch: bad arguments");
+    set_error("%s: bad arguments", what);
     return kBadArgument;
   }
   if (n_records == 0) return kOk;
-  TNBases tb;
-  for (int i = 0; i < 3; ++i) {
+  TNBases tb = {};
+  for (int i = 0; i < n_bases; ++i) {
     if (bases[i] == nullptr || strides[i] < 0 || lens[i] < 0) {
-      set_error("tedq_tn_contract_small_batch: bad arena %d", i);
+      set_error("%s: bad arena %d", what, i);
       return kBadArgument;
     }
-    tb.p[i] = static_cast<const float2*>(bases[i]);
+    tb.p[i] = static_cast<float2*>(const_cast<void*>(bases[i]));
     tb.stride[i] = strides[i];
   }
   for (int r = 0; r < n_records; ++r) {
     const int64_t* rec = records + 8 * (int64_t)r;
     TNDesc d;
     if (rec[0] < 0 || rec[0] >= n_descs || parse_desc(descs + rec[0] * (4 + 9 * 32), &d) != 0) {
-      set_error("tedq_tn_contract_small_batch: record %d: bad descriptor row %lld", r, (long long)rec[0]);
+      set_error("%s: record %d: bad descriptor row %lld", what, r, (long long)rec[0]);
       return kBadArgument;
     }
     const int nH = d.nb[0], nM = d.nb[1], nN = d.nb[2], nK = d.nb[3];
     const int64_t sa = 1ll << (nH + nM + nK), sb = 1ll << (nH + nN + nK), sc = 1ll << (nH + nM + nN);
-    const bool shapes = nH + nM + nK <= 12 && nH + nN + nK <= 12 && nH + nM + nN <= 12 && nK <= 6 && rec[6] == sc;
-    const bool in_a = rec[1] >= 0 && rec[1] < 3 && rec[2] >= 0 && rec[2] + sa <= lens[rec[1]];
-    const bool in_b = rec[3] >= 0 && rec[3] < 3 && rec[4] >= 0 && rec[4] + sb <= lens[rec[3]];
-    const bool in_c = rec[5] >= 0 && rec[5] + sc <= lens[2];
+    const int64_t ic = c_base >= 0 ? c_base : rec[7];
+    const bool shapes = nH + nM + nK <= 12 && nH + nN + nK <= 12 && nH + nM + nN <= 12 && nK <= max_k && rec[6] == sc;
+    const bool in_a = rec[1] >= 0 && rec[1] < n_bases && rec[2] >= 0 && rec[2] + sa <= lens[rec[1]];
+    const bool in_b = rec[3] >= 0 && rec[3] < n_bases && rec[4] >= 0 && rec[4] + sb <= lens[rec[3]];
+    const bool in_c = ic >= 0 && ic < n_bases && rec[5] >= 0 && rec[5] + sc <= lens[ic];
     if (!shapes || !in_a || !in_b || !in_c) {
-      set_error("tedq_tn_contract_small_batch: record %d does not fit (shape or arena bounds)", r);
+      set_error("%s: record %d does not fit (shape or arena bounds)", what, r);
       return kBadArgument;
     }
   }
   hipLaunchKernelGGL(k_tn_small_multi, dim3((unsigned)n_records, (unsigned)batch), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), tb, const_cast<float2*>(tb.p[2]), records_dev, descs_dev);
-  return check_launch("tedq_tn_contract_small_batch");
+                     static_cast<hipStream_t>(stream), tb, records_dev, descs_dev, c_base);
+  return check_launch(what);
+}
+
+// Three arenas, results in the third.
+extern "C" int tedq_tn_contract_small_batch(const void* const* bases, const int64_t* strides, const int64_t* lens,
+                                            const int64_t* records, const int64_t* records_dev, int n_records,
+                                            int64_t batch, const int32_t* descs, const int32_t* descs_dev,
+                                            int n_descs, void* stream) {
+  return launch_small("tedq_tn_contract_small_batch", bases, strides, lens, 3, records, records_dev, n_records, batch,
+                      descs, descs_dev, n_descs, 2, 6, stream);
+}
+
+// Five arenas, each record's last word naming its result's.
+extern "C" int tedq_tn_small_environments(const void* const* bases, const int64_t* strides, const int64_t* lens,
+                                          const int64_t* records, const int64_t* records_dev, int n_records,
+                                          int64_t batch, const int32_t* descs, const int32_t* descs_dev, int n_descs,
+                                          void* stream) {
+  return launch_small("tedq_tn_small_environments", bases, strides, lens, kSmallBases, records, records_dev, n_records,
+                      batch, descs, descs_dev, n_descs, -1, 12, stream);
 }
 
 // Eligibility of a forward step for tedq_tn_gate_backward (the k_tn_gate shape

@@ -655,6 +655,63 @@ class TNExecutor:
         self._small[key] = plan
         return plan
 
+    def _batch_small_backward(self, dev):
+        """Environments of the small steps one launch per tree level: on the device, with their arena."""
+        return self.small_batch and dev.type == "cuda"
+
+    def _small_env_plan(self, net):
+        """Records of the small steps' environments by tree level, last level first.  Arenas: 0 leaves,
+        1 constants, 2 small results, 3 environments of small results, 4 environments of leaves."""
+        plan = self._small_plan(net)
+        if "env" in plan:
+            return plan["env"]
+        offs = plan["offs"]
+        by_row = {int(r[0]): i for i, r in enumerate(plan["recs"])}
+        level = {}
+        for lv, (s, e) in enumerate(plan["bounds"]):
+            for i in range(s, e):
+                level[i] = lv
+
+        def operand(t):
+            if t < net.n_inputs:
+                where, o = net.leaves[t]
+                return [0 if where == "arena" else 1, o]
+            return [2, offs[t]]
+        levels = [[] for _ in plan["bounds"]]
+        for st in net.steps:
+            if st.c not in offs or not net.needs[st.c]:
+                continue
+            env = [3, offs[st.c]]
+            for row, tid, ops in ((st.bwd_a, st.a, env + operand(st.b)), (st.bwd_b, st.b, operand(st.a) + env)):
+                if row < 0 or (tid < net.n_inputs and net.leaves[tid][0] != "arena"):
+                    continue
+                out, o = (4, net.leaves[tid][1]) if tid < net.n_inputs else (3, offs[tid])
+                levels[level[by_row[st.fwd]]].append([row] + ops + [o, 1 << net.ranks[tid], out])
+        recs, bounds = [], []
+        for lv in reversed(levels):
+            if lv:
+                bounds.append((len(recs), len(recs) + len(lv)))
+                recs += lv
+        plan["env"] = {"recs": np.array(recs, dtype=np.int64).reshape(-1, 8), "bounds": bounds, "dev": {}}
+        return plan["env"]
+
+    def _small_backward(self, net, arena, env_small, env_arena, leaves, buf, B, dev):
+        """Environments of all small steps (their results' are in ``env_small`` already), level by level."""
+        env, small = self._small_env_plan(net), self._small_plan(net)
+        key = str(dev)
+        if key not in env["dev"]:
+            env["dev"][key] = torch.from_numpy(env["recs"].reshape(-1).copy()).to(dev)
+        consts, n = buf["consts"], small["len"]
+        bases = (ctypes.c_void_p * 5)(leaves.data_ptr(), consts.data_ptr(), arena.data_ptr(), env_small.data_ptr(),
+                                      env_arena.data_ptr())
+        strides = (ctypes.c_int64 * 5)(self.leaf_stride, 0, n, n, self.leaf_stride)
+        lens = (ctypes.c_int64 * 5)(self.leaf_stride, consts.numel(), n, n, self.leaf_stride)
+        for s, e in env["bounds"]:
+            hip.call("tedq_tn_small_environments", bases, strides, lens, env["recs"][s:e].ctypes.data_as(hip.c_vp),
+                     ctypes.c_void_p(env["dev"][key].data_ptr() + 64 * s), e - s, B,
+                     self._descs.ctypes.data_as(hip.c_vp), hip.ptr(buf["descs"]), self._descs.shape[0],
+                     hip.stream_handle(dev))
+
     # runs of gates on one large tensor ------------------------------------
     def _use_runs(self, dev):
         """Runs are a device path: they need the small steps' results in their arena."""
@@ -857,8 +914,8 @@ class TNExecutor:
                 if keep is not None and tid != net.root and keep(tid):
                     kept[tid] = vals[tid]
         coef = self._run_coefs(plan, small, arena, leaves, buf, B, dev) if plan is not None else None
-        if grad_runs:
-            kept["coef"] = coef
+        if keep is not None:
+            kept["arena"], kept["coef"] = arena, coef
         for s, st in enumerate(net.steps):
             if small is not None and st.c in small["offs"]:
                 continue
@@ -965,12 +1022,18 @@ class TNExecutor:
                 return seg_of.get(t, -1) != seg_of.get(net.steps[net.consumer[t]].c, -1)
         root, stored = self._forward_once(net, leaves, B, dev, keep, plan is not None)
         coef = stored.pop("coef", None)
-        env_small = None
-        if plan is not None:
-            small = self._small_plan(net)
-            env_small = torch.zeros((B, small["len"]), dtype=torch.complex64, device=dev)
         env_arena = torch.zeros((B, self.leaf_stride), dtype=torch.complex64, device=dev)
         envs = {net.root: root_env}
+        # environments of small results in one arena, their own steps batched by tree level
+        small = self._small_plan(net) if self.small_batch else None
+        small_arena = stored.pop("arena", None)
+        batched = len(segs) == 1 and self._batch_small_backward(dev) and bool(small["bounds"])
+        env_small, offs = env_arena, {}
+        if batched:
+            env_small = torch.empty((B, small["len"]), dtype=torch.complex64, device=dev)
+            offs = small["offs"]
+            if net.root in offs:
+                env_small[:, offs[net.root]:offs[net.root] + (1 << net.ranks[net.root])] = envs.pop(net.root)
         for si in range(len(segs) - 1, -1, -1):
             seg = segs[si]
             vals = dict(stored)
@@ -987,6 +1050,8 @@ class TNExecutor:
                                    buf)
             for s in reversed(seg):
                 st = net.steps[s]
+                if st.c in offs:
+                    continue
                 if plan is not None and s in plan["covered"]:
                     run = plan["last"].get(s)
                     if run is not None:
@@ -996,16 +1061,13 @@ class TNExecutor:
                         e = envs.pop(run.c, None)
                         if e is None:
                             continue
-                        e = e if isinstance(e, tuple) else (e, e.shape[1], 0)
-                        envs[run.a] = self._run_backward_passes(run, plan, coef, outs, e, env_arena, env_small, B, dev)
-                        for t in (t for ps in run.passes for op in ps.ops for t in op.factors):
-                            if t >= net.n_inputs and net.needs[t]:
-                                envs[t] = (env_small, env_small.shape[1], small["offs"][t])
+                        envs[run.a] = self._run_backward_passes(run, plan, coef, outs, (e, e.shape[1], 0), env_arena,
+                                                                env_small, B, dev)
                     continue
                 ec = envs.pop(st.c, None)
                 if ec is None:
                     continue
-                ecop = ec if isinstance(ec, tuple) else (ec, ec.shape[1], 0)
+                ecop = (ec, ec.shape[1], 0)
                 dsts = {}
                 for which, desc_row, tid in (("a", st.bwd_a, st.a), ("b", st.bwd_b, st.b)):
                     if desc_row < 0:
@@ -1015,6 +1077,8 @@ class TNExecutor:
                         if where != "arena":
                             continue
                         dsts[which] = (env_arena, self.leaf_stride, off)
+                    elif tid in offs:
+                        dsts[which] = (env_small, env_small.shape[1], offs[tid])
                     else:
                         e = torch.empty((B, 1 << net.ranks[tid]), dtype=torch.complex64, device=dev)
                         envs[tid] = e
@@ -1032,6 +1096,8 @@ class TNExecutor:
                     del vals[st.c]
             for s in seg:
                 stored.pop(net.steps[s].c, None)
+        if batched:
+            self._small_backward(net, small_arena, env_small, env_arena, leaves, buf, B, dev)
         if self.n_params:
             self._param_grad(env_arena, dmats, grad, B)
         return root

@@ -11,15 +11,18 @@ at most ~2e-7 per gate and random sign, so a few hundred gates stay below
 1e-5 of the scale; both sides of a comparison carry that.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import tedq_amd as qai
+from tedq_amd.engine import hip
 from tedq_amd.tn import runs as R
-from tedq_amd.tn.executor import TNExecutor
+from tedq_amd.tn.executor import TNExecutor, make_desc
 
-from tn_emulator import install
+from tn_emulator import contract_np, install
 
 TOL = 1e-5
 
@@ -154,7 +157,22 @@ def emulate(ex):
             e = res
         return torch.from_numpy(e.astype(np.complex64))
 
-    ex._run_coefs, ex._run_forward_passes, ex._run_backward_passes = coefs, forward, backward  # pylint: disable=protected-access
+    def small_backward(net, arena, env_small, env_arena, leaves, buf, B, dev):  # pylint: disable=unused-argument
+        env = ex._small_env_plan(net)  # pylint: disable=protected-access
+        bases = [leaves.numpy(), np.broadcast_to(buf["consts"].numpy(), (B, buf["consts"].numel())), arena.numpy(),
+                 env_small.numpy(), env_arena.numpy()]
+        for s, e in env["bounds"]:
+            for row, ia, oa, ib, ob, oc, size, ic in env["recs"][s:e]:
+                desc = ex._descs[row]  # pylint: disable=protected-access
+                nh, nm, nn, nk = (int(v) for v in desc[:4])
+                out = np.zeros((B, size), dtype=np.complex128)
+                contract_np(desc, bases[ia][:, oa:oa + (1 << (nh + nm + nk))].astype(np.complex128),
+                            bases[ib][:, ob:ob + (1 << (nh + nk + nn))].astype(np.complex128), out)
+                bases[ic][:, oc:oc + size] = out
+
+    # pylint: disable=protected-access
+    ex._run_coefs, ex._run_forward_passes, ex._run_backward_passes = coefs, forward, backward
+    ex._batch_small_backward, ex._small_backward = (lambda dev: ex.small_batch), small_backward
     return ex
 
 
@@ -306,6 +324,37 @@ def _apply(x, m, wires, n):
     idx = _index(wires, n)
     out[:, idx] = x[:, idx] @ m.T
     return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("na,nb,nk,batch", [(0, 0, 0, 1), (0, 0, 12, 2), (2, 2, 10, 3), (1, 0, 11, 1), (4, 4, 8, 2),
+                                            (6, 6, 6, 1), (11, 1, 1, 2), (3, 9, 0, 1)])
+def test_small_environments_vs_reference(na, nb, nk, batch):
+    """One step per shape: few outputs over long sums (lanes per output, k past the table), many outputs;
+    sums of 2^nk products of unit normals, fp32: 2^(nk/2) * 1e-6 of their scale."""
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(nk)
+    la = [f"m{i}" for i in range(na)] + [f"k{i}" for i in range(nk)]
+    lb = [f"k{i}" for i in range(nk)] + [f"n{i}" for i in range(nb)]
+    lc = [f"m{i}" for i in range(na)] + [f"n{i}" for i in range(nb)]
+    la, lb, lc = (list(rng.permutation(v)) for v in (la, lb, lc))
+    desc = make_desc(la, lb, lc)
+    a = rng.normal(size=(batch, 1 << (na + nk))) + 1j * rng.normal(size=(batch, 1 << (na + nk)))
+    b = rng.normal(size=(batch, 1 << (nb + nk))) + 1j * rng.normal(size=(batch, 1 << (nb + nk)))
+    ta, tb = (torch.tensor(v, dtype=torch.complex64, device=dev) for v in (a, b))
+    outs = [torch.zeros((batch, (1 << (na + nb)) + 3), dtype=torch.complex64, device=dev) for _ in range(2)]
+    ten = [ta, tb, outs[0], outs[1], outs[1]]
+    bases = (ctypes.c_void_p * 5)(*[t.data_ptr() for t in ten])
+    sizes = (ctypes.c_int64 * 5)(*[t.shape[1] for t in ten])
+    recs = np.array([[0, 0, 0, 1, 0, 3, 1 << (na + nb), 2], [0, 0, 0, 1, 0, 1, 1 << (na + nb), 4]], dtype=np.int64)
+    drecs, ddesc = torch.from_numpy(recs).to(dev), torch.from_numpy(desc).to(dev)
+    hip.call("tedq_tn_small_environments", bases, sizes, sizes, recs.ctypes.data_as(hip.c_vp), hip.ptr(drecs), 2, batch,
+             desc.ctypes.data_as(hip.c_vp), hip.ptr(ddesc), 1, hip.stream_handle(dev))
+    want = np.zeros((batch, 1 << (na + nb)), dtype=np.complex128)
+    contract_np(desc, ta.cpu().numpy().astype(np.complex128), tb.cpu().numpy().astype(np.complex128), want)
+    tol = 2 ** (nk / 2) * 1e-6 * 8
+    assert np.max(np.abs(outs[0][:, 3:].cpu().numpy() - want)) < tol
+    assert np.max(np.abs(outs[1][:, 1:-2].cpu().numpy() - want)) < tol
 
 
 @pytest.mark.gpu
