@@ -24,8 +24,9 @@ What is this module's own:
 * gradients come from the reverse contraction tree: the environment of a
   step's result gives the environments of its two operands (two more
   contraction launches), and the environments of the gate leaves give
-  d value / d theta (tedq_tn_param_grad).  Intermediates are recomputed per
-  network in the backward pass, and when they do not fit the memory cap the
+  d value / d theta (tedq_tn_param_grad).  Intermediates are kept from the
+  forward where they are small against the free memory, else recomputed per
+  network in the backward pass; when they do not fit the memory cap the
   path is cut into segments whose boundary tensors are checkpointed and whose
   insides are recomputed.
 """
@@ -945,13 +946,43 @@ class TNExecutor:
         return root, kept
 
     # ------------------------------------------------------------------
-    def run_forward(self, rows, need_grad=False):  # pylint: disable=unused-argument
-        """Contract every network for [B, P] rows.  Returns a run record for ``measure``/``run_backward``."""
+    def run_forward(self, rows, need_grad=False):
+        """Contract every network for [B, P] rows.  Returns a run record for ``measure``/``run_backward``;
+        with ``need_grad`` it holds the intermediates a backward would otherwise contract again, where
+        they are few enough (``_keeps_forward``)."""
         B = rows.shape[0]
         dev = rows.device
         leaves, dmats = self._leaves(rows)
-        roots = [self._forward_network(net, leaves, B, dev)[0] for net in self.networks]
-        return {"rows": rows, "leaves": leaves, "dmats": dmats, "roots": roots}
+        roots, kept = [], []
+        for net in self.networks:
+            if need_grad and self.n_params and self._keeps_forward(net, B, dev):
+                root, stored = self._forward_stored(net, leaves, B, dev)
+                kept.append((root, stored))
+            else:
+                root = self._forward_network(net, leaves, B, dev)[0]
+                kept.append(None)
+            roots.append(root)
+        return {"rows": rows, "leaves": leaves, "dmats": dmats, "roots": roots, "kept": kept}
+
+    def _keeps_forward(self, net, B, dev):
+        """Whether the forward of ``net`` may serve its backward: one segment, the backward's runs cover
+        (nearly) what the forward's do, so that a value alone costs no more, and the intermediates take at
+        most 1/16 of the memory that is free now, so that any number of live graphs fits."""
+        if net.sliced or dev.type != "cuda" or len(self._backward_segments(net, B, dev)[1]) > 1:
+            return False
+        if self._use_runs(dev):
+            grad, plain = (self._run_plan(net, g)["covered"] for g in (True, False))
+            if len(grad) < 0.9 * len(plain):
+                return False
+            need = self._run_bytes(net, self._run_plan(net, True), B)
+        else:
+            need = net.intermediate_elems() * B * 8
+        if need <= 64 << 20:
+            return True
+        if torch.cuda.is_current_stream_capturing():
+            return False
+        free = torch.cuda.mem_get_info(dev)[0] + torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
+        return need <= free // 16
 
     def measure(self, run):
         outs = []
@@ -990,12 +1021,12 @@ class TNExecutor:
         elems += sum(1 << net.ranks[st.c] for s, st in enumerate(net.steps) if s not in plan["covered"])
         return elems * B * 8
 
-    def _backward_network(self, net, leaves, dmats, root_env, grad, B, dev):
+    def _backward_network(self, net, leaves, dmats, root_env, grad, B, dev, kept=None):
         """Reverse contraction tree of one network; gradients are added into ``grad``.  Returns the
         network's root.  A sliced network runs forward and backward once per slice: the parameter
         gradients of the slices add up in ``grad`` and their roots are added in slice order."""
         if not net.sliced:
-            return self._backward_once(net, leaves, dmats, root_env, grad, B, dev)
+            return self._backward_once(net, leaves, dmats, root_env, grad, B, dev, kept)
         total = None
         for a in range(1 << len(net.sliced)):
             self._set_selectors(net, a, dev)
@@ -1003,24 +1034,32 @@ class TNExecutor:
             total = root.clone() if total is None else total.add_(root)
         return total
 
-    def _backward_once(self, net, leaves, dmats, root_env, grad, B, dev):
-        buf = self._buffers(dev)
+    def _backward_segments(self, net, B, dev):
+        """(run plan or None, segments of steps) of a network's backward."""
         plan = self._run_plan(net, True) if self._use_runs(dev) else None
         if plan is not None and (not plan["first"] or self._run_bytes(net, plan, B) > self._keep_budget(dev)):
             plan = None
-        segs = [list(range(len(net.steps)))] if plan is not None else self._segments(net, B, dev)
+        return plan, ([list(range(len(net.steps)))] if plan is not None else self._segments(net, B, dev))
+
+    def _forward_stored(self, net, leaves, B, dev):
+        """Forward of a backward: (root, the intermediates to keep, those that cross a segment boundary)."""
+        plan, segs = self._backward_segments(net, B, dev)
         seg_of = {}
         for si, seg in enumerate(segs):
             for s in seg:
                 seg_of[net.steps[s].c] = si
-        # forward, checkpointing the tensors that cross a segment boundary
         if len(segs) == 1:
             def keep(_t):
                 return True
         else:
             def keep(t):
                 return seg_of.get(t, -1) != seg_of.get(net.steps[net.consumer[t]].c, -1)
-        root, stored = self._forward_once(net, leaves, B, dev, keep, plan is not None)
+        return self._forward_once(net, leaves, B, dev, keep, plan is not None)
+
+    def _backward_once(self, net, leaves, dmats, root_env, grad, B, dev, kept=None):
+        buf = self._buffers(dev)
+        plan, segs = self._backward_segments(net, B, dev)
+        root, stored = kept if kept is not None else self._forward_stored(net, leaves, B, dev)
         coef = stored.pop("coef", None)
         env_arena = torch.zeros((B, self.leaf_stride), dtype=torch.complex64, device=dev)
         envs = {net.root: root_env}
@@ -1141,10 +1180,15 @@ class TNExecutor:
         B = rows.shape[0]
         dev = rows.device
         grad = torch.zeros((B, max(self.n_params, 1)), dtype=torch.float64, device=dev)
-        for spec, net, g in zip(self.specs, self.networks, grads):
+        kept = run.get("kept") or [None] * len(self.networks)
+        for i, (spec, net, g) in enumerate(zip(self.specs, self.networks, grads)):
             if g is None:
                 continue
-            self._backward_network(net, run["leaves"], run["dmats"], self._root_env(spec, g, B, net), grad, B, dev)
+            # the first backward consumes the intermediates (each freed once it has served); a second one
+            # through the same graph contracts the network again
+            stored, kept[i] = kept[i], None
+            self._backward_network(net, run["leaves"], run["dmats"], self._root_env(spec, g, B, net), grad, B, dev,
+                                   stored)
         return grad[:, :self.n_params].to(grad_dtype)
 
     def value_and_grad(self, rows, grads_out):

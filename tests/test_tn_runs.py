@@ -374,3 +374,24 @@ def test_networks_with_and_without_runs(build, args, grad, batch):
         res.append((v,) + ((ex.value_and_grad(rows, [torch.ones(batch, device=dev)])[1],) if grad else ()))
     for a, b in zip(*res):
         assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("args", [(3, 3, 2, 4, False), (4, 4, 4, 5, False), (3, 4, 3, 5, True)])
+def test_backward_from_a_kept_forward(args):
+    """A forward that keeps its intermediates serves one backward; a second backward through the same graph
+    and a forward that kept nothing contract again: the same launches on the same values, so equal bits."""
+    dev = torch.device("cuda", 0)
+    cc, npar = lattice(*args)
+    rows = rows_for(npar, 2, 5).to(dev)
+    ex = TNExecutor(cc)
+    up = [torch.ones(2, device=dev)]
+    grads = []
+    for need in (True, False):
+        run = ex.run_forward(rows, need_grad=need)
+        assert (run["kept"][0] is not None) == need
+        for _ in range(2):
+            grads.append(ex.run_backward(rows, run, ex.seed_adjoint(run, up)))
+            assert run["kept"][0] is None
+    assert all(torch.equal(grads[0], g) for g in grads[1:])
+    assert float(grads[0].abs().max()) > 1e-3
