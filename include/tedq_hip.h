@@ -98,7 +98,8 @@ int tedq_sv_pass_ragged(int adjoint, const void* dev_recs, int n_recs, int64_t t
 /* tedq_sv_apply_pass (flags bit 0 clear; lam, partials unused) or
  * tedq_sv_adjoint_pass (bit 0 set; reg_bits <= 4) for a lifted plan's program
  * (tedq_amd/engine/lift.py; stage words in csrc/sv_lift.hip), whose ops drop
- * global phases.  flags bit 1: the pass has general ops. */
+ * global phases.  flags bit 1: the pass has general ops.  Every round's table
+ * offset leaves 2^reg_bits + reg_bits + 1 entries of the row to read. */
 int tedq_sv_lift_pass(int flags, void* psi, void* lam, int64_t batch, int n_qubits, int tile_bits, int reg_bits,
                       int threads_log2, const int* dev_prog, uint64_t tile_mask, uint64_t zero_mask,
                       const void* mats, int64_t mat_stride, float* partials, int64_t partial_rows, int n_gslots,

@@ -167,10 +167,10 @@ __device__ __forceinline__ float general_grad(const float2 (&p)[R], const float2
 // multiply-adds in the adjoint, read off the generated code); behind a branch without an else they stay.
 template <int R, bool TWO, bool DAG, int KIND>
 __device__ __forceinline__ void round_rotations(float2 (&v)[R], float2 (&w)[R], int mask, int cots,
-                                                const float2* __restrict__ rt) {
+                                                const float (&qs)[5]) {
 #define CALL(B)                                             \
   if ((mask >> B) & 1) {                                    \
-    const float q = rt[B].x;                                \
+    const float q = qs[B];                                  \
     if ((cots >> B) & 1) {                                  \
       rotate_unscaled<R, B, KIND, true, DAG>(v, q);         \
       if (TWO) rotate_unscaled<R, B, KIND, true, DAG>(w, q);  \
@@ -223,8 +223,77 @@ __device__ __forceinline__ void flush_group(float (&acc)[8], float* dst, int seg
   for (int q = 0; q < 8; ++q) acc[q] = 0.f;
 }
 
+// A uniform value made to arrive in a scalar register at this point.
+__device__ __forceinline__ void pin(int& x) {
+  x = __builtin_amdgcn_readfirstlane(x);
+  asm volatile("" : "+s"(x));
+}
+__device__ __forceinline__ void pin(float& x) {
+  int i = __builtin_bit_cast(int, x);
+  pin(i);
+  x = __builtin_bit_cast(float, i);
+}
+
+// What a round's control flow needs, held in scalar registers and read one round ahead: its first words, then
+// its table row's ratios and forms (and a touch of the row's other lines).  Read where it is used, each is a
+// scalar load that the wave waits for alone, about ten in turn per round.
+template <int R>
+struct RoundHead {
+  int flags, regmask, rot, coef, sign, grads, kindp, group, group_pre, cots;
+  float q[5], line0, line1;
+  __device__ __forceinline__ void words(const int* __restrict__ st) {
+    flags = st[kLwFlags];
+    regmask = st[kLwRegmask];
+    rot = st[kLwRot];
+    coef = st[kLwCoef];
+    sign = st[kLwSign];
+    grads = st[kLwGrads];
+    kindp = st[kLwKindP];
+    group = st[kLwGroup];
+    group_pre = st[kLwGroupPre];
+  }
+  template <bool MULTI>
+  __device__ __forceinline__ void row(const float2* __restrict__ mb) {
+    const float2* d1 = mb + coef;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) q[i] = i < log2c(R) ? d1[R + i].x : 0.f;
+    cots = __builtin_bit_cast(int, d1[R + log2c(R)].x);
+    if (!MULTI) {
+      line0 = d1[0].x;
+      line1 = d1[R / 2].x;
+    }
+  }
+  // the loads are issued before here and waited for here (the row of whole-circuit tiles is the lane's own)
+  template <bool MULTI>
+  __device__ __forceinline__ void arrive() {
+    pin(flags), pin(regmask), pin(rot), pin(coef), pin(sign), pin(grads), pin(kindp), pin(group), pin(group_pre);
+    if (!MULTI) {
+      pin(cots), pin(line0), pin(line1);
+#pragma unroll
+      for (int i = 0; i < log2c(R); ++i) pin(q[i]);
+    }
+  }
+};
+
+// Touch the lines of the pass's program and of the circuit's table rows while the tile loads are in flight.
+// Both were written by another kernel, so the first scalar load of each line misses this XCD's L2 and every
+// round waits for two or three of them in turn; with one tile per circuit there is no other workgroup to hide
+// it behind.  With the reads ahead of RoundHead: first pass of 32 17-qubit circuits 60 -> 45 us forward and
+// 88 -> 71 us adjoint; 48 20-qubit forwards, 12288 tiles a pass, 3.74 -> 3.46 ms.
+__device__ __forceinline__ void warm_lines(const int* __restrict__ prog, const float2* __restrict__ mb, int nst, int row) {
+  const int t = threadIdx.x, T = blockDim.x;
+  const int words = kHdrStages + kLiftWords * nst;
+  const int c0 = prog[kHdrStages + kLwCoef], c1 = prog[kHdrStages + kLiftWords * (nst - 1) + kLwCoef];
+  const int lo = c0 < c1 ? c0 : c1, hi = (c0 < c1 ? c1 : c0) + row;
+  int w = 0;
+  float c = 0.f;
+  for (int i = 32 * t; i < words; i += 32 * T) w ^= prog[i];
+  for (int i = lo + 16 * t; i < hi; i += 16 * T) c += mb[i].x;
+  asm volatile("" ::"v"(w), "v"(c));
+}
+
 // Workgroup `blk` of a lifted pass (a tile, or G whole circuits when MULTI), forward or adjoint.  GEN: the pass
-// has general ops (without them the kernel needs 40% fewer registers and no copies around their dispatch).
+// has general ops (without them the kernel needs a third fewer registers and no copies around their dispatch).
 template <int R, bool ADJ, bool MULTI, bool GEN>
 __device__ __forceinline__ void lift_body(float2* __restrict__ psi, float2* __restrict__ lam,
                                           const int* __restrict__ prog, const float2* __restrict__ mats,
@@ -237,6 +306,8 @@ __device__ __forceinline__ void lift_body(float2* __restrict__ psi, float2* __re
   const int lane = tid & 63;
   const TileCtx c = make_ctx(a, prog, tid, MULTI, blk);
   const float2* mb = mats + (c.valid ? c.circuit : 0) * a.mat_stride;
+  const int nst = prog[2];
+  if (!MULTI) warm_lines(prog, mb, nst, R + log2c(R) + 1);
   load_tiles<R, MULTI>(psi, ldp, prog, a, tid, T, c, blk);
   if (ADJ) load_tiles<R, MULTI>(lam, ldl, prog, a, tid, T, c, blk);
   __syncthreads();
@@ -254,14 +325,19 @@ __device__ __forceinline__ void lift_body(float2* __restrict__ psi, float2* __re
   float2 vp[R], vl[R];
 #pragma unroll
   for (int m = 0; m < R; ++m) vp[m] = vl[m] = make_float2(0.f, 0.f);
-  const int nst = prog[2];
+  RoundHead<R> h;
+  h.words(prog + kHdrStages);
+  h.template row<MULTI>(mb);
   for (int s = 0; s < nst; ++s) {
     const int* st = prog + kHdrStages + kLiftWords * s;
-    const int flags = st[kLwFlags], rx = st[kLwRot] & 31, ry = (st[kLwRot] >> 8) & 31;
-    const int sb = lift_stage_base(tid, a.tT, a.k, st[kLwRegmask]);
-    const float2* d1 = mb + st[kLwCoef];
-    const float2 *rt = d1 + R, *d0 = rt + log2c(R) + 1;
-    const int cots = (rx | ry) ? __builtin_bit_cast(int, rt[log2c(R)].x) : 0;
+    const int flags = h.flags, rx = h.rot & 31, ry = (h.rot >> 8) & 31;
+    const int sb = lift_stage_base(tid, a.tT, a.k, h.regmask);
+    const float2* d1 = mb + h.coef;
+    const float2* d0 = d1 + R + log2c(R) + 1;
+    const int cots = (rx | ry) ? h.cots : 0;
+    RoundHead<R> nx;
+    const int* next = s + 1 < nst ? st + kLiftWords : st;
+    if (!GEN) nx.words(next);  // (the general ops' words and matrices need the scalar registers)
     if (!(flags & kLiftSkipRead)) {
 #pragma unroll
       for (int m = 0; m < R; ++m) {
@@ -269,18 +345,18 @@ __device__ __forceinline__ void lift_body(float2* __restrict__ psi, float2* __re
         if (ADJ) vl[m] = ldl[sb ^ st[kLwIn + m]];
       }
     }
-    const uint32_t sign = (uint32_t)st[kLwSign];
+    const uint32_t sign = (uint32_t)h.sign;
     const int ngen = GEN ? st[kLwNGen] : 0;
     if (!ADJ) {
       if (flags & kLiftD0) scale_diagonal<R, false>(vp, d0, InPlace());
-      if (rx) round_rotations<R, false, false, 0>(vp, vl, rx, cots, rt);
-      if (ry) round_rotations<R, false, false, 1>(vp, vl, ry, cots, rt);
+      if (rx) round_rotations<R, false, false, 0>(vp, vl, rx, cots, h.q);
+      if (ry) round_rotations<R, false, false, 1>(vp, vl, ry, cots, h.q);
       if (flags & kLiftD1) scale_diagonal<R, false>(vp, d1, InPlace());
       if (flags & kLiftScale) scale_all<R>(vp, d1->x);
       for (int o = 0; o < ngen; ++o) general_op<R, false>(vp, vl, prog + st[kLwGen] + 8 * o, mb);
       if (sign) round_signs<R>(vp, sign);
     } else {
-      const int gr = st[kLwGrads], kindp = st[kLwKindP];
+      const int gr = h.grads, kindp = h.kindp;
       if (sign) {
         round_signs<R>(vp, sign);
         round_signs<R>(vl, sign);
@@ -304,21 +380,23 @@ __device__ __forceinline__ void lift_body(float2* __restrict__ psi, float2* __re
         scale_all<R>(vp, f);
         scale_all<R>(vl, f);
       }
-      if (rx) round_rotations<R, true, true, 0>(vp, vl, rx, cots, rt);
-      if (ry) round_rotations<R, true, true, 1>(vp, vl, ry, cots, rt);
+      if (rx) round_rotations<R, true, true, 0>(vp, vl, rx, cots, h.q);
+      if (ry) round_rotations<R, true, true, 1>(vp, vl, ry, cots, h.q);
       // (a rotation commutes with its generator: its gradient may be taken before it, where no factor is pending)
       if (gr & rx) rotation_grads<R, kGradX>(vp, vl, gr & rx, acc);
       if (gr & ry) rotation_grads<R, kGradY>(vp, vl, gr & ry, acc);
-      if (st[kLwGroup] >= 0) flush_group(acc, pbase + (int64_t)st[kLwGroup] * a.np * 8, seg, lane, writer);
-      if (st[kLwGroupPre] >= 0) {
+      if (h.group >= 0) flush_group(acc, pbase + (int64_t)h.group * a.np * 8, seg, lane, writer);
+      if (h.group_pre >= 0) {
         phase_grads<R>(vp, vl, (gr >> 16) & 31, (kindp >> 8) & 31, acc);
-        flush_group(acc, pbase + (int64_t)st[kLwGroupPre] * a.np * 8, seg, lane, writer);
+        flush_group(acc, pbase + (int64_t)h.group_pre * a.np * 8, seg, lane, writer);
       }
       if (flags & kLiftD0) {
         scale_diagonal<R, true>(vp, d0, InPlace());
         scale_diagonal<R, true>(vl, d0, InPlace());
       }
     }
+    if (GEN) nx.words(next);
+    nx.template row<MULTI>(mb);
     if (!(flags & kLiftSkipWrite)) {
 #pragma unroll
       for (int m = 0; m < R; ++m) {
@@ -326,6 +404,8 @@ __device__ __forceinline__ void lift_body(float2* __restrict__ psi, float2* __re
         if (ADJ) ldl[sb ^ st[kLwOut + m]] = vl[m];
       }
     }
+    nx.template arrive<MULTI>();
+    h = nx;
     if (flags & kLiftBarrier) __syncthreads();
   }
   store_tiles<R, MULTI>(psi, ldp, prog, a, tid, T, c, blk);

@@ -283,7 +283,8 @@ def _round_words(rd, r, slots, adjoint, skip_read, skip_write, barrier, pdep, sw
             if slots[si].gslot >= 0:
                 grads[1 + i] |= 1 << b
                 kindp[i] |= int(slots[si].pauli[0] == 3) << b
-    w[W_COEF], w[W_SIGN] = rd.coef, rd.sign
+    # a round of general ops only has no table row: the kernel, which reads ahead, finds row 0
+    w[W_COEF], w[W_SIGN] = (rd.coef if rd.pre or rd.rot or rd.post else 0), rd.sign
     w[W_GRADS] = grads[0] | grads[1] << 8 | grads[2] << 16
     w[W_KINDP] = kindp[0] | kindp[1] << 8
     w[W_GROUP], w[W_GROUP_PRE] = rd.group, rd.group_pre

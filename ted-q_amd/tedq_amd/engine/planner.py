@@ -356,7 +356,8 @@ def build_plan(n, units, n_params, const_pool, k_max=12, r=4, coalesce_bits=3, s
         from .lift import assign_rounds  # pylint: disable=import-outside-toplevel
         rounds, mat_off, gslot = assign_rounds(passes, slots, r, lift == "fwd")
         return Plan(n=n, k=k, r=r, passes=passes, slots=slots, const_pool=np.asarray(const_pool, dtype=np.complex128),
-                    n_params=n_params, n_gslots=gslot, mat_stride=max(mat_off, 1), specialize=True, rounds=rounds)
+                    n_params=n_params, n_gslots=gslot, mat_stride=max(mat_off, (1 << r) + r + 1), specialize=True,
+                    rounds=rounds)
     mat_off = 0
     for s in slots:
         s.mat_off = mat_off

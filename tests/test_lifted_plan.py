@@ -332,3 +332,30 @@ def test_lifted_plan_makes_user_matrices_dense_and_keeps_registers_between_round
     flags = [int(words[LF.HDR_STAGES + LF.STAGE_WORDS * i]) for i in range(len(rounds))]
     assert all(f & LF.SKIP_WRITE for f in flags[:-1])
     assert flags[-1] & (LF.SKIP_READ | LF.SKIP_WRITE | LF.BARRIER) == LF.SKIP_READ | LF.BARRIER
+
+
+@pytest.mark.parametrize("last", ["matrix", "controlled", "rotation"])
+def test_every_round_leaves_a_whole_row_to_read_ahead(last):
+    """The kernels read 2^r + r + 1 table entries of the next round before they know whether it uses them: also
+    for rounds of general ops only (no row of their own), the last of them at the end of the table."""
+    rng = np.random.default_rng(2)
+    u = np.linalg.qr(rng.normal(size=(4, 4)) + 1j * rng.normal(size=(4, 4)))[0]
+
+    def circuit_def():
+        qai.Unitary(u, qubits=[0, 1])
+        qai.RY(0.4, qubits=[2])
+        if last == "matrix":
+            qai.Unitary(u, qubits=[2, 3])
+            qai.Unitary(u, qubits=[1, 2])
+        elif last == "controlled":
+            qai.CRX(0.3, qubits=[0, 3])
+        return qai.expval(qai.PauliZ(qubits=[0]))
+    n, units, npar, pool = lower_circuit(qai.Circuit(circuit_def, 4).compilecircuit(backend="pytorch"))
+    for lift in ("fwd", True):
+        for k, r in ((4, 4), (3, 2), (2, 1)):
+            plan = build_plan(n, units, npar, list(pool), k_max=k, r=r, lift=lift)
+            enc = P.encode_plan(plan)
+            for off in list(enc.fwd_offsets) + list(enc.adj_offsets):
+                for s in range(int(enc.prog[off + 2])):
+                    st = enc.prog[off + P.HDR_STAGES + LF.STAGE_WORDS * s:]
+                    assert 0 <= st[LF.W_COEF] <= plan.mat_stride - ((1 << r) + r + 1)
