@@ -302,6 +302,7 @@ class _Network:
         self.lay = lay
         self.ranks = [len(x) for x in lay]
         self.needs = needs
+        self._elems = None
         # step index of the consumer of every tensor id
         self.consumer = {}
         for s, st in enumerate(self.steps):
@@ -310,7 +311,9 @@ class _Network:
         self.root = self.n_inputs + len(self.steps) - 1
 
     def intermediate_elems(self):
-        return sum(1 << self.ranks[st.c] for st in self.steps)
+        if self._elems is None:
+            self._elems = sum(1 << self.ranks[st.c] for st in self.steps)
+        return self._elems
 
 
 def _external_paths(cc, paths):
@@ -956,8 +959,8 @@ class TNExecutor:
         roots, kept = [], []
         for net in self.networks:
             if need_grad and self.n_params and self._keeps_forward(net, B, dev):
-                root, stored = self._forward_stored(net, leaves, B, dev)
-                kept.append((root, stored))
+                kept.append(self._forward_stored(net, leaves, B, dev))
+                root = kept[-1][0]
             else:
                 root = self._forward_network(net, leaves, B, dev)[0]
                 kept.append(None)
@@ -1017,9 +1020,11 @@ class TNExecutor:
 
     def _run_bytes(self, net, plan, B):
         """Bytes of intermediates the backward keeps when the runs store one tensor per pass."""
-        elems = sum(len(run.passes) << run.wires for run in plan["first"].values())
-        elems += sum(1 << net.ranks[st.c] for s, st in enumerate(net.steps) if s not in plan["covered"])
-        return elems * B * 8
+        if "elems" not in plan:
+            elems = sum(len(run.passes) << run.wires for run in plan["first"].values())
+            elems += sum(1 << net.ranks[st.c] for s, st in enumerate(net.steps) if s not in plan["covered"])
+            plan["elems"] = elems
+        return plan["elems"] * B * 8
 
     def _backward_network(self, net, leaves, dmats, root_env, grad, B, dev, kept=None):
         """Reverse contraction tree of one network; gradients are added into ``grad``.  Returns the
@@ -1042,7 +1047,7 @@ class TNExecutor:
         return plan, ([list(range(len(net.steps)))] if plan is not None else self._segments(net, B, dev))
 
     def _forward_stored(self, net, leaves, B, dev):
-        """Forward of a backward: (root, the intermediates to keep, those that cross a segment boundary)."""
+        """Forward of a backward: (root, the intermediates that cross a segment boundary, run plan, segments)."""
         plan, segs = self._backward_segments(net, B, dev)
         seg_of = {}
         for si, seg in enumerate(segs):
@@ -1054,12 +1059,11 @@ class TNExecutor:
         else:
             def keep(t):
                 return seg_of.get(t, -1) != seg_of.get(net.steps[net.consumer[t]].c, -1)
-        return self._forward_once(net, leaves, B, dev, keep, plan is not None)
+        return self._forward_once(net, leaves, B, dev, keep, plan is not None) + (plan, segs)
 
     def _backward_once(self, net, leaves, dmats, root_env, grad, B, dev, kept=None):
         buf = self._buffers(dev)
-        plan, segs = self._backward_segments(net, B, dev)
-        root, stored = kept if kept is not None else self._forward_stored(net, leaves, B, dev)
+        root, stored, plan, segs = kept if kept is not None else self._forward_stored(net, leaves, B, dev)
         coef = stored.pop("coef", None)
         env_arena = torch.zeros((B, self.leaf_stride), dtype=torch.complex64, device=dev)
         envs = {net.root: root_env}
