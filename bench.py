@@ -418,15 +418,28 @@ def tn_leg(c4=True, c3=True):
 
 
 def tn_bound_s(ex, batch, with_grad):
-    """Roofline time of the executed contraction steps: per step the larger of 8 flops per complex
+    """Roofline time of the executed contraction: per step the larger of 8 flops per complex
     multiply-add at the 157.3 TFLOP/s FP32 matrix peak and its operand + result bytes at 8 TB/s
-    (forward steps, plus both environment steps of the backward when ``with_grad``)."""
+    (forward steps, plus both environment steps of the backward when ``with_grad``).  A pass of a run
+    counts once: the large tensor read and written (backward: its result and environment read, the
+    environment written) and the multiply-adds of the pass's matrices (backward: three such products)."""
     total = 0.0
     for net in ex.networks:
-        for st in net.steps:
+        # pylint: disable=protected-access
+        plan = ex._run_plan(net, with_grad) if ex.run_passes and ex.small_batch else {"covered": (), "first": {}}
+        for run in plan["first"].values():
+            size = batch * 2.0 ** run.wires
+            for ps in run.passes:
+                flops = sum(8.0 * size * 2 ** max(2, len(op.wires)) for op in ps.ops)
+                total += max(flops / 157.3e12, 16.0 * size / 8e12)
+                if with_grad:
+                    total += max(3 * flops / 157.3e12, 24.0 * size / 8e12)
+        for s, st in enumerate(net.steps):
+            if s in plan["covered"]:
+                continue
             rows = [st.fwd] + ([r for r in (st.bwd_a, st.bwd_b) if r >= 0] if with_grad else [])
             for r in rows:
-                nh, nm, nn, nk = (int(v) for v in ex._descs[r][:4])  # pylint: disable=protected-access
+                nh, nm, nn, nk = (int(v) for v in ex._descs[r][:4])
                 flops = 8.0 * batch * 2.0 ** (nh + nm + nn + nk)
                 byts = 8.0 * batch * (2.0 ** (nh + nm + nk) + 2.0 ** (nh + nn + nk) + 2.0 ** (nh + nm + nn))
                 total += max(flops / 157.3e12, byts / 8e12)
