@@ -380,7 +380,9 @@ class TNExecutor:
         self.run_passes = True
         self._small = {}
         self._run_plans = {}
-        self._leaf_unitary = {idx: _unitary_gate(op) for idx, op in cc._operators.items()}  # pylint: disable=protected-access
+        # rank of the leaf that holds a unitary gate's whole matrix (0: not unitary)
+        self._unitary_rank = {idx: 2 * len(op.qubits) if _unitary_gate(op) else 0
+                              for idx, op in cc._operators.items()}  # pylint: disable=protected-access
         ext = _external_paths(cc, paths)
         # diagonal reduction (the reference's tn_simplify, by gate type): the wires along which gates are
         # diagonal (all of a diagonal gate's, the controls of a controlled gate) are merged into
@@ -731,7 +733,9 @@ class TNExecutor:
 
         def leaf_unitary(source, rank):
             if source[0] in ("gate", "adj"):
-                return self._leaf_unitary[source[1]]
+                # a reduced leaf (a diagonal, a matrix per control value) maps no half of its indices to the
+                # other, also where its rank is even
+                return rank == self._unitary_rank[source[1]]
             if source[0] == "obs":
                 m = np.asarray(net.measurement.obs[source[1]].matrix)
             elif source[0] == "obsmat":

@@ -306,8 +306,9 @@ def encode_run(run, source, lay):
 
 
 class Unitarity:
-    """Which gate-sized tensors are unitary maps between two halves of their indices: gate leaves by their
-    operator, small products when one factor's whole contact lies in one half of each operand."""
+    """Which gate-sized tensors are unitary maps between two halves of their indices: whole gate leaves by their
+    operator (``leaf_unitary(source, rank)``: False for reduced ones), small products when one factor's whole
+    contact lies in one half of each operand."""
 
     def __init__(self, net, leaf_unitary):
         self.net = net

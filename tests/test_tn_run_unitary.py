@@ -1,0 +1,143 @@
+"""Which gates the backward of runs may undo (tedq_amd.tn.runs.Unitarity).
+
+The backward of a run recovers an op's input as M^H of its result, so every
+matrix of a backward run has to be unitary.  Diagonal reduction stores a
+diagonal gate as its diagonal and a controlled gate per control value: such a
+leaf is no map between the halves of its indices, whatever its rank.
+
+Tolerance of M^H M = 1: the matrices are products of complex64 entries, whose
+rounding of 6e-8 per entry gives at most 4 * 8 * 6e-8 = 2e-6 for an 8 x 8
+matrix.  Gradients: as in test_tn_runs.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import tedq_amd as qai
+from tedq_amd.tn import runs as R
+from tedq_amd.tn.executor import TNExecutor
+
+from test_tn_runs import TOL, emulate, rows_for
+from tn_emulator import install
+
+UNITARY_TOL = 2e-6
+_DIAG = np.diag(np.exp(1j * np.array([0.1, 0.7, -0.4, 0.9])))
+
+
+def grid(n, width):
+    return [(q, q + 1) for q in range(n - 1) if (q + 1) % width] + [(q, q + width) for q in range(n - width)]
+
+
+def circuit(gate, n, width, layers, obs):
+    """Layers of RX on every qubit, then ``gate`` on every bond of a grid (Toffoli: also on the next qubit)."""
+    bonds = grid(n, width)
+    trained = gate in ("CRZ", "ControlledPhaseShift")
+    n_params = layers * (n + (len(bonds) if trained else 0))
+
+    def cd(*p):
+        it = iter(p)
+        for _ in range(layers):
+            for q in range(n):
+                qai.RX(next(it), qubits=[q])
+            for a, b in bonds:
+                if gate == "Unitary":
+                    qai.Unitary(_DIAG, qubits=[a, b])
+                elif gate == "Toffoli":
+                    qai.Toffoli(qubits=[a, b, next(q % n for q in (b + 1, b + 2) if q % n not in (a, b))])
+                else:
+                    getattr(qai, gate)(*([next(it)] if trained else []), qubits=[a, b])
+        return [qai.expval(qai.PauliZ(qubits=[obs]))]
+    return qai.Circuit(cd, n, *([0.1] * n_params)).compilecircuit(backend="pytorch", tn_mode=True), n_params
+
+
+class _Offered(R.Unitarity):
+    """Counts the ops with a reduced leaf that the selection was asked about; no such leaf has halves."""
+    reduced = 0
+
+    def __init__(self, net, leaf_unitary):
+        super().__init__(net, leaf_unitary)
+        for t, src in enumerate(net.sources):
+            if self._reduced(t):
+                assert self.halves(t) is None, (src, net.lay[t])
+
+    def _reduced(self, t):
+        src = self.net.sources[t]
+        return src[0] in ("gate", "adj") and len(self.net.lay[t]) < 2 * self.qubits[src[1]]
+
+    def _leaves(self, tid):
+        if tid < self.net.n_inputs:
+            return [tid]
+        st = self.maker[tid]
+        return self._leaves(st.a) + self._leaves(st.b)
+
+    def __call__(self, tid, summed):
+        _Offered.reduced += any(self._reduced(t) for t in self._leaves(tid))
+        return super().__call__(tid, summed)
+
+
+def _backward_matrices(ex, rows):
+    """The matrices of every backward run, and the number of forward run ops (``ex`` emulated)."""
+    leaves, _ = ex._leaves(rows)  # pylint: disable=protected-access
+    buf, mats, forward = ex._buffers(None), [], 0  # pylint: disable=protected-access
+    for net in ex.networks:
+        small = ex._small_plan(net)  # pylint: disable=protected-access
+        arena = torch.zeros((1, small["len"]), dtype=torch.complex64)
+        ex._small_levels(small, arena, leaves, buf, 1, None)  # pylint: disable=protected-access
+        plan = ex._run_plan(net, True)  # pylint: disable=protected-access
+        mats += ex._run_coefs(plan, small, arena, leaves, buf, 1, None)[0]  # pylint: disable=protected-access
+        forward += len(ex._run_plan(net, False)["ops"])  # pylint: disable=protected-access
+    return mats, forward
+
+
+# default options (the reduction is chosen by the path model), then reduction forced; the last two have merged
+# controls of one wire (rank 3: the small steps kept to gate merges) and of two (rank 4)
+@pytest.mark.parametrize("gate,n,width,layers,obs,forced", [
+    ("CRZ", 19, 4, 3, 9, False), ("CRZ", 17, 4, 4, 8, False), ("CRZ", 21, 5, 3, 11, False),
+    ("ControlledPhaseShift", 19, 4, 3, 9, False), ("CZ", 19, 4, 3, 9, False), ("Unitary", 17, 4, 4, 8, False),
+    ("CRZ", 16, 4, 4, 8, True), ("ControlledPhaseShift", 15, 5, 4, 7, True), ("CNOT", 17, 4, 3, 8, True),
+    ("Toffoli", 12, 4, 4, 6, True)])
+def test_backward_runs_hold_unitary_matrices(gate, n, width, layers, obs, forced, monkeypatch):
+    cc, n_params = circuit(gate, n, width, layers, obs)
+    rows = rows_for(n_params, 1, 3)
+    opts = {"diagonal_reduction": True} if forced else {}
+    ex, plain = emulate(TNExecutor(cc, **opts)), install(TNExecutor(cc, **opts))
+    assert ex.simplify
+    if forced:
+        ex.SMALL_RANK = 6
+    _Offered.qubits = {idx: len(op.qubits) for idx, op in cc._operators.items()}  # pylint: disable=protected-access
+    _Offered.reduced = 0
+    monkeypatch.setattr(R, "Unitarity", _Offered)
+    mats, forward = _backward_matrices(ex, rows)
+    assert forward, "the network has no run"
+    assert _Offered.reduced, "no op with a reduced leaf was offered to the backward"
+    for m in mats:
+        assert np.max(np.abs(m.conj().T @ m - np.eye(len(m)))) < UNITARY_TOL
+    up = [torch.ones(1)]
+    monkeypatch.undo()
+    (v, g), (vw, gw) = ex.value_and_grad(rows, up), plain.value_and_grad(rows, up)
+    assert abs(float(v[0][0] - vw[0][0])) < TOL
+    assert float((g - gw).abs().max()) < TOL * max(1.0, float(gw.abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gate,n,width,layers,obs,batch", [
+    ("CRZ", 19, 4, 3, 9, 2), ("CRZ", 17, 4, 4, 8, 1), ("ControlledPhaseShift", 17, 4, 4, 8, 2), ("CZ", 19, 4, 3, 9, 1),
+    ("Unitary", 17, 4, 4, 8, 2), ("Toffoli", 17, 4, 4, 8, 2)])
+def test_gradients_with_and_without_runs(gate, n, width, layers, obs, batch):
+    """Default options on the device: values and gradients of the runs against the steps, where the backward
+    has runs beside steps that it must not undo (Toffoli: unreduced, all of its large steps in runs)."""
+    cc, n_params = circuit(gate, n, width, layers, obs)
+    dev = torch.device("cuda", 0)
+    rows = rows_for(n_params, batch, 5).to(dev)
+    ex = TNExecutor(cc)
+    assert all(len(ex._run_plan(ex.networks[0], grad)["ops"]) for grad in (False, True))  # pylint: disable=protected-access
+    up, res = [torch.ones(batch, device=dev)], []
+    for on in (True, False):
+        ex.run_passes = on
+        v, g = ex.value_and_grad(rows, up)
+        run = ex.run_forward(rows, need_grad=True)
+        res.append((v[0], g, ex.measure(run)[0], ex.run_backward(rows, run, ex.seed_adjoint(run, up))))
+    for a, b in zip(*res):
+        assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
+    assert float(res[0][1].abs().max()) > 1e-3
