@@ -88,10 +88,17 @@ def diagonal_wires(op):
     return 0
 
 
+# Deviation from M M^H = 1 (Frobenius) up to which the backward of a run may recover an op's input as M^H of its
+# result.  The deviations of a pass's gates add up, a repeated matrix's with the same sign: a pass has up to 32 ops,
+# each a product of gates, so a bound near the rounding of complex64 (1e-7, a matrix given in single precision)
+# could put several 1e-6 into a gradient.  Matrices given in double precision are within 1e-15.
+_UNITARY_TOL = 1e-9
+
+
 def _unitary_matrix(m):
     m = np.asarray(m, dtype=np.complex128)
     m = m.reshape(int(round(np.sqrt(m.size))), -1)
-    return bool(np.max(np.abs(m @ m.conj().T - np.eye(m.shape[0]))) < 1e-6)
+    return bool(np.linalg.norm(m @ m.conj().T - np.eye(m.shape[0])) < _UNITARY_TOL)
 
 
 def _unitary_gate(op):

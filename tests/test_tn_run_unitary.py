@@ -120,6 +120,34 @@ def test_backward_runs_hold_unitary_matrices(gate, n, width, layers, obs, forced
     assert float((g - gw).abs().max()) < TOL * max(1.0, float(gw.abs().max()))
 
 
+def test_a_matrix_near_a_unitary_one_is_not_undone():
+    """Four copies per layer of a matrix that is unitary but for a factor of 1 + 4.5e-7: undone, each adds 9e-7
+    of the gradients of the gates before it.  The two paths round about 800 results to complex64 with random
+    sign: 800^(1/2) * 6e-8 = 1.7e-6 of the gradients' scale, within 4e-6."""
+    n, layers, copies = 10, 8, 4
+    near = (1 + 4.5e-7) * np.array([[np.cos(0.3), -np.sin(0.3)], [np.sin(0.3), np.cos(0.3)]])
+
+    def cd(*p):
+        it = iter(p)
+        for _ in range(layers):
+            for q in range(n):
+                qai.RX(next(it), qubits=[q])
+            for q in range(n - 1):
+                qai.CNOT(qubits=[q, q + 1])
+            for q in list(range(n)) * copies:
+                qai.Unitary(near, qubits=[q])
+        return [qai.expval(qai.PauliZ(qubits=[n // 2]))]
+    cc = qai.Circuit(cd, n, *([0.1] * (layers * n))).compilecircuit(backend="pytorch", tn_mode=True,
+                                                                     tn_simplify=False)
+    rows, up = rows_for(layers * n, 1, 3), [torch.ones(1)]
+    ex, plain = emulate(TNExecutor(cc, trials=())), install(TNExecutor(cc, trials=()))
+    ex.SMALL_RANK = 4
+    assert ex._run_plan(ex.networks[0], False)["first"], "the network has no run"  # pylint: disable=protected-access
+    (v, g), (vw, gw) = ex.value_and_grad(rows, up), plain.value_and_grad(rows, up)
+    assert abs(float(v[0][0] - vw[0][0])) < 4e-6
+    assert float((g - gw).abs().max()) < 4e-6 * float(gw.abs().max())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("gate,n,width,layers,obs,batch", [
     ("CRZ", 19, 4, 3, 9, 2), ("CRZ", 17, 4, 4, 8, 1), ("ControlledPhaseShift", 17, 4, 4, 8, 2), ("CZ", 19, 4, 3, 9, 1),
