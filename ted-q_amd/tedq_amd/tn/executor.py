@@ -799,18 +799,14 @@ class TNExecutor:
     def _run_forward_passes(self, run, plan, coef, x, B, dev, keep):
         """The results of a run's passes (only the last one unless ``keep``)."""
         outs = []
-        spare = None
-        for i, ps in enumerate(run.passes):
-            out = spare
-            if out is None or keep or i == len(run.passes) - 1:
-                out = torch.empty((B, 1 << run.wires), dtype=torch.complex64, device=dev)
+        for ps in run.passes:
+            out = torch.empty((B, 1 << run.wires), dtype=torch.complex64, device=dev)
             hip.call("tedq_tn_run_pass", ctypes.c_void_p(x[0].data_ptr() + 8 * x[2]), x[1], hip.ptr(out), out.shape[1],
                      B, ps.words.ctypes.data_as(hip.c_vp), *self._op_rows(plan, ps, dev), hip.ptr(coef),
                      plan["coef"], hip.stream_handle(dev))
-            spare = x[0] if i > 0 and not keep else None
             x = (out, out.shape[1], 0)
-            outs.append(out)
-        return outs if keep else outs[-1:]
+            outs = outs + [out] if keep else [out]
+        return outs
 
     def _run_backward_passes(self, run, plan, coef, outs, env, env_arena, env_small, B, dev):
         """Environment of a run's input from its result's, the gates' environments going to the arenas."""
@@ -937,12 +933,19 @@ class TNExecutor:
             if plan is not None and s in plan["covered"]:
                 run = plan["first"].get(s)
                 if run is not None:
-                    outs = self._run_forward_passes(run, plan, coef, self._operand(net, vals, run.a, leaves, buf), B,
-                                                    dev, grad_runs)
-                    vals[run.c] = outs[-1]
+                    x, outs = self._operand(net, vals, run.a, leaves, buf), []
+                    vals.pop(run.a, None)
+                    # one pass per call: two large tensors at a time, as step by step (the input goes after the
+                    # first pass)
+                    for part in run.parts():
+                        out = self._run_forward_passes(part, plan, coef, x, B, dev, False)[0]
+                        x = (out, out.shape[1], 0)
+                        if grad_runs:
+                            outs.append(out)
+                    vals[run.c] = out
+                    del x, out
                     if grad_runs:
                         kept["run", s] = outs
-                    vals.pop(run.a, None)
                 continue
             out = torch.empty((B, 1 << net.ranks[st.c]), dtype=torch.complex64, device=dev)
             vals[st.c] = out

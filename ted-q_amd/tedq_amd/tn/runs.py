@@ -61,6 +61,10 @@ class Run:
     out_bit: list      # address bit of every wire in the result
     passes: list
 
+    def parts(self):
+        """The run pass by pass."""
+        return [Run(self.a, self.c, self.steps, self.wires, self.out_bit, [ps]) for ps in self.passes]
+
 
 def _symbols(lay, st, big, small):
     sb, ss, sc = set(lay[big]), set(lay[small]), set(lay[st.c])
