@@ -33,6 +33,8 @@ What is this module's own:
 
 import ctypes
 import math
+import threading
+import weakref
 from dataclasses import dataclass
 
 import numpy as np
@@ -104,6 +106,28 @@ def _unitary_matrix(m):
 def _unitary_gate(op):
     """Parametrised gates are unitary for every value; a constant matrix is what the user gave."""
     return op.num_params > 0 or _unitary_matrix(op.matrix)
+
+
+class _Kept:
+    """Intermediates of one network's forward, waiting for its backward (``stored``: _forward_stored)."""
+
+    def __init__(self, executor, device, nbytes):
+        self.executor, self.device, self.nbytes = id(executor), str(device), nbytes
+        self.stored = None
+
+
+# Every forward that waits, of all executors: their bytes are bounded together, however many networks, graphs and
+# executors are alive.  Up to _KEPT_FREELY per device without a look at the free memory (which a stream that is
+# being captured must not ask for), beyond it 1/16 of what would be free without them.
+_KEPT = weakref.WeakSet()
+_KEPT_LOCK = threading.Lock()
+_KEPT_FREELY = 64 << 20
+_KEPT_SHARE = 16
+
+
+def _kept_bytes(device, executor=None):
+    """Bytes of the waiting forwards on a device, of one executor or of all (_KEPT_LOCK held)."""
+    return sum(k.nbytes for k in _KEPT if k.device == str(device) and executor in (None, k.executor))
 
 
 _NO_SRC = -2 ** 31
@@ -376,8 +400,9 @@ class TNExecutor:
         from .path import SEARCH_TRIALS  # pylint: disable=import-outside-toplevel
         trials = SEARCH_TRIALS if trials is None else trials
         self.n = cc._num_qubits  # pylint: disable=protected-access
-        # bytes of intermediates the backward may keep before it checkpoints segments and recomputes
-        # them; None: 40% of the device's memory (115 GB on a 288 GB MI355X), 64 GiB off the GPU
+        # bytes of intermediates the backward may keep (those of forwards that wait for their backward
+        # included) before it checkpoints segments and recomputes them; None: 40% of the device's memory
+        # (115 GB on a 288 GB MI355X), 64 GiB off the GPU
         self.max_bytes = max_bytes
         # forward: run the small steps of each tree level in one launch (tedq_tn_contract_small_batch)
         self.small_batch = True
@@ -966,40 +991,49 @@ class TNExecutor:
     def run_forward(self, rows, need_grad=False):
         """Contract every network for [B, P] rows.  Returns a run record for ``measure``/``run_backward``;
         with ``need_grad`` it holds the intermediates a backward would otherwise contract again, where
-        they are few enough (``_keeps_forward``)."""
+        they are few enough (``_keep_forward``)."""
         B = rows.shape[0]
         dev = rows.device
         leaves, dmats = self._leaves(rows)
         roots, kept = [], []
         for net in self.networks:
-            if need_grad and self.n_params and self._keeps_forward(net, B, dev):
-                kept.append(self._forward_stored(net, leaves, B, dev))
-                root = kept[-1][0]
+            held = self._keep_forward(net, B, dev) if need_grad and self.n_params else None
+            if held is not None:
+                held.stored = self._forward_stored(net, leaves, B, dev)
+                root = held.stored[0]
             else:
                 root = self._forward_network(net, leaves, B, dev)[0]
-                kept.append(None)
+            kept.append(held)
             roots.append(root)
         return {"rows": rows, "leaves": leaves, "dmats": dmats, "roots": roots, "kept": kept}
 
-    def _keeps_forward(self, net, B, dev):
-        """Whether the forward of ``net`` may serve its backward: one segment, the backward's runs cover
-        (nearly) what the forward's do, so that a value alone costs no more, and the intermediates take at
-        most 1/16 of the memory that is free now, so that any number of live graphs fits."""
+    def _keep_forward(self, net, B, dev):
+        """A place for the forward of ``net`` to wait for its backward, or None: there has to be one segment,
+        the backward's runs have to cover (nearly) what the forward's do, so that a value alone costs no more,
+        and the intermediates have to fit the budget of all waiting forwards (_KEPT) and ``max_bytes``."""
         if net.sliced or dev.type != "cuda" or len(self._backward_segments(net, B, dev)[1]) > 1:
-            return False
+            return None
         if self._use_runs(dev):
             grad, plain = (self._run_plan(net, g)["covered"] for g in (True, False))
             if len(grad) < 0.9 * len(plain):
-                return False
+                return None
             need = self._run_bytes(net, self._run_plan(net, True), B)
         else:
             need = net.intermediate_elems() * B * 8
-        if need <= 64 << 20:
-            return True
-        if torch.cuda.is_current_stream_capturing():
-            return False
-        free = torch.cuda.mem_get_info(dev)[0] + torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
-        return need <= free // 16
+        with _KEPT_LOCK:
+            live = _kept_bytes(dev)
+            if live + need > _KEPT_FREELY:
+                if torch.cuda.is_current_stream_capturing():
+                    return None
+                free = (torch.cuda.mem_get_info(dev)[0] + torch.cuda.memory_reserved(dev)
+                        - torch.cuda.memory_allocated(dev))
+                if live + need > (free + live) // _KEPT_SHARE:
+                    return None
+            if self.max_bytes is not None and _kept_bytes(dev, id(self)) + need > self.max_bytes:
+                return None
+            held = _Kept(self, dev, need)
+            _KEPT.add(held)
+        return held
 
     def measure(self, run):
         outs = []
@@ -1019,11 +1053,17 @@ class TNExecutor:
 
     # ------------------------------------------------------------------
     def _keep_budget(self, dev=None):
+        """Bytes of intermediates a backward may keep: the cap less this executor's waiting forwards."""
         if self.max_bytes is not None:
-            return self.max_bytes
-        if dev is not None and dev.type == "cuda":
-            return int(0.4 * torch.cuda.get_device_properties(dev).total_memory)
-        return 64 << 30
+            cap = self.max_bytes
+        elif dev is not None and dev.type == "cuda":
+            cap = int(0.4 * torch.cuda.get_device_properties(dev).total_memory)
+        else:
+            cap = 64 << 30
+        if dev is None:
+            return cap
+        with _KEPT_LOCK:
+            return cap - _kept_bytes(dev, id(self))
 
     def _segments(self, net, B, dev=None):
         total = net.intermediate_elems() * B * 8
@@ -1204,9 +1244,9 @@ class TNExecutor:
                 continue
             # the first backward consumes the intermediates (each freed once it has served); a second one
             # through the same graph contracts the network again
-            stored, kept[i] = kept[i], None
+            held, kept[i] = kept[i], None
             self._backward_network(net, run["leaves"], run["dmats"], self._root_env(spec, g, B, net), grad, B, dev,
-                                   stored)
+                                   held.stored if held is not None else None)
         return grad[:, :self.n_params].to(grad_dtype)
 
     def value_and_grad(self, rows, grads_out):
