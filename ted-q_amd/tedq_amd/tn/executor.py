@@ -651,6 +651,14 @@ class TNExecutor:
             return t
         return t, t.shape[1], 0
 
+    @staticmethod
+    def _table(plan, name, dev):
+        """Device copy of a plan's records, made on first use."""
+        key = str(dev)
+        if key not in plan["dev"]:
+            plan["dev"][key] = torch.from_numpy(plan[name].reshape(-1).copy()).to(dev)
+        return plan["dev"][key]
+
     # small steps, batched per tree level ---------------------------------
     SMALL_RANK = 12     # operands and result
     SMALL_SUM_BITS = 6  # summed indices
@@ -736,9 +744,7 @@ class TNExecutor:
     def _small_backward(self, net, arena, env_small, env_arena, leaves, buf, B, dev):
         """Environments of all small steps (their results' are in ``env_small`` already), level by level."""
         env, small = self._small_env_plan(net), self._small_plan(net)
-        key = str(dev)
-        if key not in env["dev"]:
-            env["dev"][key] = torch.from_numpy(env["recs"].reshape(-1).copy()).to(dev)
+        drecs = self._table(env, "recs", dev)
         consts, n = buf["consts"], small["len"]
         bases = (ctypes.c_void_p * 5)(leaves.data_ptr(), consts.data_ptr(), arena.data_ptr(), env_small.data_ptr(),
                                       env_arena.data_ptr())
@@ -746,7 +752,7 @@ class TNExecutor:
         lens = (ctypes.c_int64 * 5)(self.leaf_stride, consts.numel(), n, n, self.leaf_stride)
         for s, e in env["bounds"]:
             hip.call("tedq_tn_small_environments", bases, strides, lens, env["recs"][s:e].ctypes.data_as(hip.c_vp),
-                     ctypes.c_void_p(env["dev"][key].data_ptr() + 64 * s), e - s, B,
+                     ctypes.c_void_p(drecs.data_ptr() + 64 * s), e - s, B,
                      self._descs.ctypes.data_as(hip.c_vp), hip.ptr(buf["descs"]), self._descs.shape[0],
                      hip.stream_handle(dev))
 
@@ -802,18 +808,22 @@ class TNExecutor:
         self._run_plans[key] = plan
         return plan
 
+    def _run_tables(self, net, dev):
+        """Op tables of both of a network's run plans on the device: which one a pass uses depends on the memory
+        budget at the time, and a stream that is being captured takes no copies from the host."""
+        for grad in (False, True):
+            self._table(self._run_plan(net, grad), "ops", dev)
+
     def _run_coefs(self, plan, small, arena, leaves, buf, B, dev):
         """The op matrices of every run of a network, one launch: [B, plan coef]."""
-        key = str(dev)
-        if key not in plan["dev"]:
-            plan["dev"][key] = torch.from_numpy(plan["ops"].reshape(-1).copy()).to(dev)
+        ops = self._table(plan, "ops", dev)
         consts = buf["consts"]
         coef = torch.empty((B, plan["coef"]), dtype=torch.complex64, device=dev)
         bases = (ctypes.c_void_p * 3)(leaves.data_ptr(), consts.data_ptr(), arena.data_ptr())
         strides = (ctypes.c_int64 * 3)(self.leaf_stride, 0, small["len"])
         lens = (ctypes.c_int64 * 3)(self.leaf_stride, consts.numel(), small["len"])
         hip.call("tedq_tn_run_coefs", bases, strides, lens, plan["ops"].ctypes.data_as(hip.c_vp),
-                 hip.ptr(plan["dev"][key]), len(plan["ops"]), hip.ptr(coef), plan["coef"], B, hip.stream_handle(dev))
+                 hip.ptr(ops), len(plan["ops"]), hip.ptr(coef), plan["coef"], B, hip.stream_handle(dev))
         return coef
 
     @staticmethod
@@ -857,10 +867,7 @@ class TNExecutor:
 
     def _small_levels(self, plan, arena, leaves, buf, B, dev):
         """Run a plan's levels in order, one launch each, results into ``arena`` [B, plan len]."""
-        key = str(dev)
-        if key not in plan["dev"]:
-            plan["dev"][key] = torch.from_numpy(plan["recs"].reshape(-1).copy()).to(dev)
-        drecs = plan["dev"][key]
+        drecs = self._table(plan, "recs", dev)
         consts = buf["consts"]
         bases = (ctypes.c_void_p * 3)(leaves.data_ptr(), consts.data_ptr(), arena.data_ptr())
         strides = (ctypes.c_int64 * 3)(self.leaf_stride, 0, plan["len"])
@@ -939,6 +946,8 @@ class TNExecutor:
         kept = {}
         small = self._small_plan(net) if self.small_batch else None
         plan = self._run_plan(net, grad_runs) if (keep is None or grad_runs) and self._use_runs(dev) else None
+        if plan is not None:
+            self._run_tables(net, dev)
         if plan is not None and not plan["first"]:
             plan = None
         arena = leaves
@@ -1124,7 +1133,10 @@ class TNExecutor:
         # environments of small results in one arena, their own steps batched by tree level
         small = self._small_plan(net) if self.small_batch else None
         small_arena = stored.pop("arena", None)
-        batched = len(segs) == 1 and self._batch_small_backward(dev) and bool(small["bounds"])
+        batched = self._batch_small_backward(dev) and bool(small["bounds"])
+        if batched and dev.type == "cuda":
+            self._table(self._small_env_plan(net), "recs", dev)      # (like _run_tables)
+        batched = batched and len(segs) == 1
         env_small, offs = env_arena, {}
         if batched:
             env_small = torch.empty((B, small["len"]), dtype=torch.complex64, device=dev)

@@ -121,6 +121,26 @@ def test_a_captured_forward_asks_for_no_memory_info(monkeypatch):
     assert ex._keep_forward(ex.networks[0], 1, dev) is None  # pylint: disable=protected-access
 
 
+def test_both_run_plans_are_on_the_device_together(monkeypatch):
+    """Whether a forward waits for its backward decides which of the two run plans it uses, and may differ between
+    an eager call and the same call under capture, when no table may be copied to the device any more."""
+    cc, n_params = lattice(4, 4, 4, 5, False)
+    ex = TNExecutor(cc, trials=())
+    net = ex.networks[0]
+    monkeypatch.setattr(ex, "_use_runs", lambda dev: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(hip, "stream_handle", lambda dev: None)
+    monkeypatch.setattr(hip, "call", lambda name, *args: None)
+    rows = rows_for(n_params, 1, 3)
+    leaves, _ = ex._leaves(rows)  # pylint: disable=protected-access
+    ex._forward_stored(net, leaves, 1, rows.device)  # pylint: disable=protected-access
+    copied = []
+    monkeypatch.setattr(torch, "from_numpy", copied.append)
+    ex._forward_network(net, leaves, 1, rows.device)  # pylint: disable=protected-access
+    ex._forward_stored(net, leaves, 1, rows.device)  # pylint: disable=protected-access
+    assert not copied
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("need_free", [False, True])
 def test_memory_between_forward_and_backward(need_free, monkeypatch):
@@ -155,3 +175,39 @@ def test_memory_between_forward_and_backward(need_free, monkeypatch):
         g = ex.run_backward(rows[i], runs[i], ex.seed_adjoint(runs[i], up))
         assert float((g - want[i]).abs().max()) < 1e-5 * max(1.0, float(want[i].abs().max()))
     assert all(k is None for run in runs for k in run["kept"])
+
+
+@pytest.mark.gpu
+def test_capture_of_a_forward_that_may_not_wait(monkeypatch):
+    """Value and gradient captured after an eager call that kept its forward, with the budget used up: every replay
+    equals the eager result of its parameters."""
+    cc, n_params = lattice(4, 4, 4, 5, False)
+    dev = torch.device("cuda", 0)
+    ex = TNExecutor(cc)
+    rows = rows_for(n_params, 2, 5).to(dev)
+    up = [torch.ones(2, device=dev)]
+
+    def step():
+        run = ex.run_forward(rows, need_grad=True)
+        return ex.measure(run)[0], ex.run_backward(rows, run, ex.seed_adjoint(run, up)), run["kept"]
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        held = ex._keep_forward(ex.networks[0], 2, dev)  # pylint: disable=protected-access
+        assert held is not None
+        del held
+        step()
+        torch.cuda.synchronize()
+        monkeypatch.setattr(X, "_KEPT_FREELY", 0)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            value, grad, _ = step()
+    monkeypatch.undo()
+    torch.cuda.synchronize()
+    for seed in (7, 8, 9):
+        rows.copy_(rows_for(n_params, 2, seed))
+        want_v, want_g, _ = step()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((value - want_v).abs().max()) < 1e-5
+        assert float((grad - want_g).abs().max()) < 1e-5 * max(1.0, float(want_g.abs().max()))
