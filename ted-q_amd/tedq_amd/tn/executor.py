@@ -113,7 +113,7 @@ class _Kept:
 
     def __init__(self, executor, device, nbytes):
         self.executor, self.device, self.nbytes = id(executor), str(device), nbytes
-        self.stored = None
+        self.stored = self.stream = None
 
 
 # Every forward that waits, of all executors: their bytes are bounded together, however many networks, graphs and
@@ -1008,6 +1008,7 @@ class TNExecutor:
         for net in self.networks:
             held = self._keep_forward(net, B, dev) if need_grad and self.n_params else None
             if held is not None:
+                held.stream = hip.stream_handle(dev).value
                 held.stored = self._forward_stored(net, leaves, B, dev)
                 root = held.stored[0]
             else:
@@ -1257,6 +1258,10 @@ class TNExecutor:
             # the first backward consumes the intermediates (each freed once it has served); a second one
             # through the same graph contracts the network again
             held, kept[i] = kept[i], None
+            # each intermediate goes back to the stream it was allocated on when its last use is issued: a backward
+            # on another stream would still be reading it, and contracts again
+            if held is not None and held.stream != hip.stream_handle(dev).value:
+                held = None
             self._backward_network(net, run["leaves"], run["dmats"], self._root_env(spec, g, B, net), grad, B, dev,
                                    held.stored if held is not None else None)
         return grad[:, :self.n_params].to(grad_dtype)

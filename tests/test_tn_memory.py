@@ -211,3 +211,29 @@ def test_capture_of_a_forward_that_may_not_wait(monkeypatch):
         torch.cuda.synchronize()
         assert float((value - want_v).abs().max()) < 1e-5
         assert float((grad - want_g).abs().max()) < 1e-5 * max(1.0, float(want_g.abs().max()))
+
+
+@pytest.mark.gpu
+def test_a_backward_on_another_stream_contracts_again(monkeypatch):
+    """The intermediates belong to the forward's stream; a backward elsewhere, after waiting for the forward, leaves
+    them alone and gives the same gradient."""
+    cc, n_params = lattice(4, 4, 4, 5, False)
+    dev = torch.device("cuda", 0)
+    ex = TNExecutor(cc)
+    rows, up = rows_for(n_params, 2, 5).to(dev), [torch.ones(2, device=dev)]
+    run = ex.run_forward(rows, need_grad=True)
+    want = ex.run_backward(rows, run, ex.seed_adjoint(run, up))
+    run = ex.run_forward(rows, need_grad=True)
+    used, backward = [], ex._backward_network  # pylint: disable=protected-access
+
+    def traced(*args):
+        used.append(args[-1])
+        return backward(*args)
+    monkeypatch.setattr(ex, "_backward_network", traced)
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(other):
+        got = ex.run_backward(rows, run, ex.seed_adjoint(run, up))
+    torch.cuda.synchronize()
+    assert used == [None]
+    assert torch.equal(got, want)
