@@ -18,7 +18,7 @@ import tedq_amd as qai
 from tedq_amd.tn import runs as R
 from tedq_amd.tn.executor import TNExecutor
 
-from test_tn_runs import TOL, emulate, rows_for
+from test_tn_runs import TOL, chain, emulate, lattice, rows_for
 from tn_emulator import install
 
 UNITARY_TOL = 2e-6
@@ -166,6 +166,34 @@ def test_gradients_with_and_without_runs(gate, n, width, layers, obs, batch):
         v, g = ex.value_and_grad(rows, up)
         run = ex.run_forward(rows, need_grad=True)
         res.append((v[0], g, ex.measure(run)[0], ex.run_backward(rows, run, ex.seed_adjoint(run, up))))
+    for a, b in zip(*res):
+        assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
+    assert float(res[0][1].abs().max()) > 1e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("build,args,backward,batch", [
+    (chain, (40, 8, True), True, 1), (lattice, (3, 5, 5, 7, False), True, 2), (lattice, (4, 5, 6, 9, True), True, 1),
+    (lattice, (5, 5, 3, 12, True), False, 2)])
+def test_networks_that_have_runs(build, args, backward, batch):
+    """Networks whose runs are known to exist (forward only in the last, where reduction leaves the backward
+    none): values, gradients, and the gradient from a kept forward against the steps."""
+    cc, n_params = build(*args)
+    dev = torch.device("cuda", 0)
+    rows = rows_for(n_params, batch, 11).to(dev)
+    ex = TNExecutor(cc)
+    net = ex.networks[0]
+    covered = [len(ex._run_plan(net, grad)["covered"]) for grad in (False, True)]  # pylint: disable=protected-access
+    assert covered[0] > 20 and (covered[1] > 20) == backward
+    up, res = [torch.ones(batch, device=dev)], []
+    for on in (True, False):
+        ex.run_passes = on
+        v, g = ex.value_and_grad(rows, up)
+        run = ex.run_forward(rows, need_grad=True)
+        if on and covered[1] >= 0.9 * covered[0]:
+            assert run["kept"][0] is not None
+        res.append((v[0], g, ex.measure(run)[0], ex.run_backward(rows, run, ex.seed_adjoint(run, up)),
+                    ex.measure(ex.run_forward(rows))[0]))
     for a, b in zip(*res):
         assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
     assert float(res[0][1].abs().max()) > 1e-3
