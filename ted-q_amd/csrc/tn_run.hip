@@ -453,15 +453,35 @@ __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __rest
 // carries a spectator bit, which is summed here).
 // 1024 threads: the workgroups' rows are 128 B apart reads of one matrix, a
 // chain of loads per thread (39 us per pass with 256 threads and no unrolling).
+// A rotation rounded to fp32 is a unitary matrix times 1 + O(1e-7): M^H M = s,
+// the same for every row, so undoing the ops o, o + 1, ... of the pass left
+// their inputs scaled by the product of their s, which no sum averages out.  It
+// is divided out here in fp64 (16 qubits, 6 layers of a lattice: 1.11 times the
+// error of stored inputs without it).
 __global__ void __launch_bounds__(1024) k_tn_run_env(const float* __restrict__ part, int n_wg, int coef,
-                                                     const int32_t* __restrict__ ops, float2* env0, int64_t bs0,
-                                                     float2* env1, int64_t bs1) {
-  __shared__ double sum[1024];
+                                                     const int32_t* __restrict__ ops, int n_ops,
+                                                     const float2* __restrict__ m, int64_t m_bs, float2* env0,
+                                                     int64_t bs0, float2* env1, int64_t bs1) {
+  __shared__ double sum[1024], scale[16];
   __shared__ float2 val[64];
   const int32_t* w = ops + (int64_t)blockIdx.x * kOpWords;
   if (w[W_EBASE] < 0) return;
   const int64_t b = blockIdx.y;
   const int t = threadIdx.x, a = w[W_ARITY], size = 2 << (2 * a), off = 2 * (w[W_COEF] - ops[W_COEF]);
+  // sum of s - 1 = tr(M^H M) / D - 1 over the ops, a wave per op (first order: the squares are below 1e-11)
+  double dev = 0.0;
+  for (int o = blockIdx.x + (t >> 6); o < n_ops; o += 16) {
+    const int32_t* wo = ops + o * kOpWords;
+    const int ao = wo[W_ARITY], e = t & 63;
+    if (e < (1 << (2 * ao))) {
+      const float2 v = m[b * m_bs + wo[W_COEF] + e];
+      dev += ((double)v.x * v.x + (double)v.y * v.y) / (1 << ao);
+    }
+    if (e == 0) dev -= 1.0;
+  }
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) dev += __shfl_xor(dev, h, 64);
+  if ((t & 63) == 0) scale[t >> 6] = dev;
   const int step = 1024 / size;
   const float* p = part + b * n_wg * (int64_t)(2 * coef) + off + (t & (size - 1));
   double s = 0.0;
@@ -471,7 +491,9 @@ __global__ void __launch_bounds__(1024) k_tn_run_env(const float* __restrict__ p
   __syncthreads();
   if (t < size) {
     for (int q = 1; q < step; ++q) s += sum[q * size + t];
-    reinterpret_cast<float*>(val)[t] = (float)s;
+    double d = 0.0;
+    for (int q = 0; q < 16; ++q) d += scale[q];
+    reinterpret_cast<float*>(val)[t] = (float)(s - d * s);
   }
   __syncthreads();
   const int32_t* f = w + W_F;
@@ -695,7 +717,8 @@ extern "C" int tedq_tn_run_backward(const void* c, int64_t c_bs, const void* ec,
   const int rc = check_launch("tedq_tn_run_backward");
   if (rc != kOk) return rc;
   hipLaunchKernelGGL(k_tn_run_env, dim3((unsigned)P.n_ops, (unsigned)batch), dim3(1024), 0, st,
-                     static_cast<const float*>(workspace), groups, P.coef, ops_dev, static_cast<float2*>(env0), bs0,
+                     static_cast<const float*>(workspace), groups, P.coef, ops_dev, P.n_ops,
+                     static_cast<const float2*>(coef), coef_bs, static_cast<float2*>(env0), bs0,
                      static_cast<float2*>(env1), bs1);
   return check_launch("tedq_tn_run_backward(env)");
 }

@@ -18,7 +18,7 @@ import tedq_amd as qai
 from tedq_amd.tn import runs as R
 from tedq_amd.tn.executor import TNExecutor
 
-from test_tn_runs import TOL, chain, emulate, lattice, rows_for
+from test_tn_runs import TOL, _apply, _rows, chain, emulate, lattice, rows_for
 from tn_emulator import install
 
 UNITARY_TOL = 2e-6
@@ -197,3 +197,58 @@ def test_networks_that_have_runs(build, args, backward, batch):
     for a, b in zip(*res):
         assert float((a - b).abs().max()) < TOL * max(1.0, float(b.abs().max()))
     assert float(res[0][1].abs().max()) > 1e-3
+
+
+def _rounded_rotation(sign):
+    """The RY in fp32, of many angles, whose c^2 + s^2 is furthest from 1 on one side."""
+    a = np.linspace(0.1, 1.4, 4001)
+    c, s = np.cos(a).astype(np.float32).astype(np.float64), np.sin(a).astype(np.float32).astype(np.float64)
+    i = int(np.argmax(sign * (c * c + s * s - 1)))
+    assert sign * (c[i] ** 2 + s[i] ** 2 - 1) > 5e-8
+    return np.array([[c[i], -s[i]], [s[i], c[i]]], dtype=np.complex128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("n,ops,batch", [(9, 32, 2), (12, 32, 1), (14, 20, 2)])
+def test_rounding_of_the_undone_matrices_does_not_add_up(sign, n, ops, batch):
+    """One pass of rotations that are all rounded to the same side of unitary: undone, each scales the recovered
+    input by up to 1 + 1e-7.  Against float64 with the stored inputs, environments whose sums do not cancel:
+    3e-7 of their size (rounding of the results 6e-8, of sums of at most 16 terms per lane with random sign, and
+    of random signs elsewhere); left in, the factors give up to 32 * 1e-7."""
+    dev, rng = torch.device("cuda", 0), np.random.default_rng(n)
+    m = _rounded_rotation(sign)
+    chain_ops = []
+    for k in range(ops):
+        w = k % min(n, 9)
+        op = R.Op([f"i{k}"], [f"o{k}"], [k], [], [w])
+        op.in_wire, op.out_wire = {f"i{k}": w}, {f"o{k}": w}
+        chain_ops.append(op)
+    run = R.Run(0, 1, [], n, list(range(n)), R._split_passes(chain_ops, n))  # pylint: disable=protected-access
+    assert len(run.passes) == 1
+    rows = R.encode_run(run, lambda t: (0, 4 * t), [list(reversed(op.outs)) + list(reversed(op.ins)) for op in chain_ops])
+    for row in rows:
+        row[8], row[9] = 0, row[13]
+    plan = {"ops": np.array(rows, dtype=np.int32), "coef": int(run.passes[0].words[3]), "dev": {}}
+    ex = TNExecutor.__new__(TNExecutor)
+    ex.leaf_stride = 4 * ops
+    leaves = torch.tensor(np.tile(m.reshape(-1), (batch, ops)), dtype=torch.complex64, device=dev)
+    buf = {"consts": torch.zeros(2, dtype=torch.complex64, device=dev)}
+    # pylint: disable=protected-access
+    coef = ex._run_coefs(plan, {"len": 4 * ops}, leaves, leaves, buf, batch, dev)
+    x = rng.normal(size=(batch, 1 << n)) + 1j * rng.normal(size=(batch, 1 << n))
+    tx = torch.tensor(x, dtype=torch.complex64, device=dev)
+    outs = ex._run_forward_passes(run, plan, coef, (tx, tx.shape[1], 0), batch, dev, True)
+    te = outs[-1].conj().resolve_conj().contiguous()
+    envs = [torch.zeros((batch, 4 * ops), dtype=torch.complex64, device=dev) for _ in range(2)]
+    ex._run_backward_passes(run, plan, coef, outs, (te, te.shape[1], 0), envs[0], envs[1], batch, dev)
+    states = [tx.cpu().numpy().astype(np.complex128)]
+    for op in run.passes[0].ops:
+        states.append(_apply(states[-1], m, op.wires, n))
+    env, got = te.cpu().numpy().astype(np.complex128), envs[0].cpu().numpy()
+    for k in range(ops - 1, -1, -1):
+        op = run.passes[0].ops[k]
+        want = np.einsum("brq,brk->bqk", _rows(env, op.wires, n), _rows(states[k], op.wires, n)).reshape(batch, 4)
+        t = op.factors[0]
+        assert np.max(np.abs(got[:, 4 * t:4 * t + 4] - want)) < 3e-7 * np.max(np.abs(want)), k
+        env = _apply(env, m.T, op.wires, n)
