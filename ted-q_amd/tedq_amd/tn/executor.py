@@ -815,15 +815,16 @@ class TNExecutor:
             self._table(self._run_plan(net, grad), "ops", dev)
 
     def _run_coefs(self, plan, small, arena, leaves, buf, B, dev):
-        """The op matrices of every run of a network, one launch: [B, plan coef]."""
+        """The op matrices of every run of a network: [B, plan coef] and one more entry per op (the scale of its
+        rounding, tedq_tn_run_coefs)."""
         ops = self._table(plan, "ops", dev)
         consts = buf["consts"]
-        coef = torch.empty((B, plan["coef"]), dtype=torch.complex64, device=dev)
+        coef = torch.empty((B, plan["coef"] + len(plan["ops"])), dtype=torch.complex64, device=dev)
         bases = (ctypes.c_void_p * 3)(leaves.data_ptr(), consts.data_ptr(), arena.data_ptr())
         strides = (ctypes.c_int64 * 3)(self.leaf_stride, 0, small["len"])
         lens = (ctypes.c_int64 * 3)(self.leaf_stride, consts.numel(), small["len"])
         hip.call("tedq_tn_run_coefs", bases, strides, lens, plan["ops"].ctypes.data_as(hip.c_vp),
-                 hip.ptr(ops), len(plan["ops"]), hip.ptr(coef), plan["coef"], B, hip.stream_handle(dev))
+                 hip.ptr(ops), len(plan["ops"]), hip.ptr(coef), coef.shape[1], B, hip.stream_handle(dev))
         return coef
 
     @staticmethod
@@ -838,7 +839,7 @@ class TNExecutor:
             out = torch.empty((B, 1 << run.wires), dtype=torch.complex64, device=dev)
             hip.call("tedq_tn_run_pass", ctypes.c_void_p(x[0].data_ptr() + 8 * x[2]), x[1], hip.ptr(out), out.shape[1],
                      B, ps.words.ctypes.data_as(hip.c_vp), *self._op_rows(plan, ps, dev), hip.ptr(coef),
-                     plan["coef"], hip.stream_handle(dev))
+                     coef.shape[1], hip.stream_handle(dev))
             x = (out, out.shape[1], 0)
             outs = outs + [out] if keep else [out]
         return outs
@@ -857,7 +858,7 @@ class TNExecutor:
             ex = env[0] if owned else torch.empty((B, 1 << run.wires), dtype=torch.complex64, device=dev)
             hip.call("tedq_tn_run_backward", hip.ptr(c), c.shape[1],
                      ctypes.c_void_p(env[0].data_ptr() + 8 * env[2]), env[1], hip.ptr(ex), ex.shape[1], B, words,
-                     *self._op_rows(plan, ps, dev), hip.ptr(coef), plan["coef"], hip.ptr(env_arena),
+                     *self._op_rows(plan, ps, dev), hip.ptr(coef), coef.shape[1], hip.ptr(env_arena),
                      self.leaf_stride, self.leaf_stride, hip.ptr(env_small), env_small.shape[1], env_small.shape[1],
                      hip.ptr(ws), ws_bytes, hip.stream_handle(dev))
             # only the last pass changes the layout, so the others may write over the environment they read

@@ -252,3 +252,51 @@ def test_rounding_of_the_undone_matrices_does_not_add_up(sign, n, ops, batch):
         t = op.factors[0]
         assert np.max(np.abs(got[:, 4 * t:4 * t + 4] - want)) < 3e-7 * np.max(np.abs(want)), k
         env = _apply(env, m.T, op.wires, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("products,singles,batch", [(1, 0, 1), (40, 3, 2), (300, 0, 2)])
+def test_rounding_of_products_does_not_add_up(products, singles, batch):
+    """Matrices of ops that are the product of two rotations, all the same and so all rounded alike, then ops of one
+    factor: the scale of the roundings, |M| against the product in float64, is balanced in one op, whose own
+    rounding remains (6e-8 at most); the matrices themselves are right to 4 roundings and the balance."""
+    dev, arena = torch.device("cuda", 0), []
+    rng = np.random.default_rng(3)
+
+    def rotation(a):
+        return np.array([[np.cos(a), -np.sin(a)], [np.sin(a), np.cos(a)]]).astype(np.complex64).astype(np.complex128)
+    cands = [(rotation(a), rotation(b)) for a, b in rng.uniform(0.2, 1.3, size=(2000, 2))]
+
+    def scale(m, p):
+        return 0.5 * (np.sum(np.abs(m) ** 2) / np.sum(np.abs(p) ** 2) - 1)
+    a, b = max(cands, key=lambda f: scale((f[1] @ f[0]).astype(np.complex64).astype(np.complex128), f[1] @ f[0]))
+    assert scale((b @ a).astype(np.complex64).astype(np.complex128), b @ a) > 3e-8
+    ops, lay = [], []
+    for k in range(products + singles):
+        names, w = [len(lay)] + ([len(lay) + 1] if k < products else []), k % 9
+        lay += [["x", f"i{k}"], [f"o{k}", "x"]] if k < products else [[f"o{k}", f"i{k}"]]
+        arena += [a, b] if k < products else [a]
+        op = R.Op([f"i{k}"], [f"o{k}"], names, ["x"] if k < products else [], [w])
+        op.in_wire, op.out_wire = {f"i{k}": w}, {f"o{k}": w}
+        ops.append(op)
+    rows = [R.encode_op(op, list(range(9)), lambda t: (0, 4 * t), lay) for op in ops]
+    for k, row in enumerate(rows):
+        row[7] = 16 * k
+    plan = {"ops": np.array(rows, dtype=np.int32), "coef": 16 * len(ops), "dev": {}}
+    ex = TNExecutor.__new__(TNExecutor)
+    ex.leaf_stride = 4 * len(arena)
+    leaves = torch.tensor(np.tile(np.concatenate([m.reshape(-1) for m in arena]), (batch, 1)), dtype=torch.complex64,
+                          device=dev)
+    buf = {"consts": torch.zeros(2, dtype=torch.complex64, device=dev)}
+    coef = ex._run_coefs(plan, {"len": 4 * len(arena)}, leaves, leaves, buf, batch, dev)  # pylint: disable=protected-access
+    got = coef.cpu().numpy().astype(np.complex128)
+    for e in range(batch):
+        total = 0.0
+        for k in range(len(ops)):
+            m = got[e, 16 * k:16 * k + 16].reshape(4, 4)
+            p = b @ a if k < products else a
+            want = np.kron(np.eye(2), p) if ops[k].wires[0] == 0 else np.kron(p, np.eye(2))
+            # (the spectator slot is the lowest other one)
+            assert np.max(np.abs(m - want)) < 4 * 6e-8 + products * 6e-8 * (k == products - 1)
+            total += scale(m, want)
+        assert abs(total) <= 6e-8
