@@ -412,6 +412,7 @@ class TNExecutor:
         self.run_passes = True
         self._small = {}
         self._run_plans = {}
+        self._run_tabled = set()
         # rank of the leaf that holds a unitary gate's whole matrix (0: not unitary)
         self._unitary_rank = {idx: 2 * len(op.qubits) if _unitary_gate(op) else 0
                               for idx, op in cc._operators.items()}  # pylint: disable=protected-access
@@ -811,8 +812,10 @@ class TNExecutor:
     def _run_tables(self, net, dev):
         """Op tables of both of a network's run plans on the device: which one a pass uses depends on the memory
         budget at the time, and a stream that is being captured takes no copies from the host."""
-        for grad in (False, True):
-            self._table(self._run_plan(net, grad), "ops", dev)
+        if (id(net), dev) not in self._run_tabled:
+            for grad in (False, True):
+                self._table(self._run_plan(net, grad), "ops", dev)
+            self._run_tabled.add((id(net), dev))
 
     def _run_coefs(self, plan, small, arena, leaves, buf, B, dev):
         """The op matrices of every run of a network: [B, plan coef] and one more entry per op (the scale of its
