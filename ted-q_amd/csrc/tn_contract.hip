@@ -448,10 +448,16 @@ static TNPermPlan perm_plan(const TNDesc& d, int a_tensor) {
 // count, C base id; a base id selects one of the (pointer, batch stride) pairs
 // passed by value.  One launch per tree level: a 5x5 lattice's backward had
 // 1172 launches of 4 us (a launch's own latency) for these steps, now 25 of 13 us.
-constexpr int kSmallBases = 5;
+// ENV: the environments.  The forward's sums have at most 2^6 terms and go to one
+// arena; its steps are short, so it does without lanes, eight sums and the larger
+// tables (four rows of a 40-qubit chain of 4 layers: 300 us of its launches, 437
+// with lanes, 323 with the eight sums).
+constexpr int kSmallBases = 5, kSmallResults = 2, kSmallSumBits = 6;
+template <bool ENV>
 struct TNBases {
-  float2* p[kSmallBases];
-  int64_t stride[kSmallBases];
+  static constexpr int kCount = ENV ? kSmallBases : kSmallResults + 1;
+  float2* p[kCount];
+  int64_t stride[kCount];
 };
 
 __device__ __forceinline__ void mul_add(float2& acc, float2 x, float2 y) {
@@ -459,11 +465,13 @@ __device__ __forceinline__ void mul_add(float2& acc, float2 x, float2 y) {
   acc.y = fmaf(x.x, y.y, fmaf(x.y, y.x, acc.y));
 }
 
-__global__ void __launch_bounds__(256) k_tn_small_multi(TNBases bases, const int64_t* __restrict__ recs,
-                                                        const int32_t* __restrict__ descs, int c_base) {
+template <bool ENV>
+__global__ void __launch_bounds__(256) k_tn_small_multi(TNBases<ENV> bases, const int64_t* __restrict__ recs,
+                                                        const int32_t* __restrict__ descs) {
+  constexpr int kTab = ENV ? kTabBits : kSmallSumBits;
   __shared__ TNShared d;
   __shared__ signed char mapA[32], mapB[32];
-  __shared__ uint32_t tka[1 << kTabBits], tkb[1 << kTabBits];
+  __shared__ uint32_t tka[1 << kTab], tkb[1 << kTab];
   const int64_t* rec = recs + 8 * (int64_t)blockIdx.x;
   const int row = (int)rec[0];
   load_desc(d, descs + (int64_t)row * (4 + 9 * 32));
@@ -471,58 +479,63 @@ __global__ void __launch_bounds__(256) k_tn_small_multi(TNBases bases, const int
   const int nH = d.nb[0], nM = d.nb[1], nN = d.nb[2], nK = d.nb[3];
   const int rc = nH + nM + nN;
   const int t = threadIdx.x;
-  const int kt = nK < kTabBits ? nK : kTabBits;
+  const int kt = nK < kTab ? nK : kTab;
   for (int k = t; k < (1 << kt); k += 256) {
     tka[k] = scat(d, AK, kt, k);
     tkb[k] = scat(d, BK, kt, k);
   }
   __syncthreads();
   const int64_t b = blockIdx.y;
-  const int ia = (int)rec[1], ib = (int)rec[3], ic = c_base >= 0 ? c_base : (int)rec[7];
+  const int ia = (int)rec[1], ib = (int)rec[3], ic = ENV ? (int)rec[7] : kSmallResults;
   const float2* a = bases.p[ia] + b * bases.stride[ia] + rec[2];
   const float2* bp = bases.p[ib] + b * bases.stride[ib] + rec[4];
   float2* c = bases.p[ic] + b * bases.stride[ic] + rec[5];
   const int n_out = (int)rec[6];
   int lpo = 0;
-  while (lpo < 6 && lpo < nK && (n_out << lpo) < 256) ++lpo;
+  if (ENV)
+    while (lpo < 6 && lpo < nK && (n_out << lpo) < 256) ++lpo;
   // whole groups of lanes leave the loop together, so the shuffles see every lane of a group
   for (int i = t; i < (n_out << lpo); i += 256) {
     const int o = i >> lpo;
     const uint32_t oa = via_map(mapA, rc, (uint32_t)o), ob = via_map(mapB, rc, (uint32_t)o);
-    // eight sums per lane, added pairwise like the lanes': one sum of up to 2^6 terms in turn has twice the
-    // rounding (12-qubit gradients: 1.10 times the error of 64 lanes per output), and eight loads are in flight
-    float2 acc[8];
+    const int k0 = i & ((1 << lpo) - 1);
+    float2 acc = make_float2(0.f, 0.f);
+    if (ENV && kt - lpo >= 3) {
+      // eight sums per lane, added pairwise like the lanes': one sum of up to 2^8 terms in turn has several
+      // times the rounding (12-qubit gradients: 1.10 times the error of 64 lanes per output), and eight loads
+      // are in flight
+      float2 part[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc[u] = make_float2(0.f, 0.f);
-    for (int kh = 0; kh < (1 << (nK - kt)); ++kh) {
-      uint32_t ha = oa, hb = ob;
-      for (int j = kt; j < nK; ++j) {
-        const uint32_t bit = ((uint32_t)kh >> (j - kt)) & 1u;
-        ha |= bit << d.pos[AK][j];
-        hb |= bit << d.pos[BK][j];
-      }
-      const int k0 = i & ((1 << lpo) - 1);
-      if (kt - lpo >= 3) {
+      for (int u = 0; u < 8; ++u) part[u] = make_float2(0.f, 0.f);
+      for (int kh = 0; kh < (1 << (nK - kt)); ++kh) {
+        uint32_t ha = oa, hb = ob;
+        for (int j = kt; j < nK; ++j) {
+          const uint32_t bit = ((uint32_t)kh >> (j - kt)) & 1u;
+          ha |= bit << d.pos[AK][j];
+          hb |= bit << d.pos[BK][j];
+        }
         for (int k = k0; k < (1 << kt); k += 8 << lpo) {
 #pragma unroll
-          for (int u = 0; u < 8; ++u) mul_add(acc[u], a[ha | tka[k + (u << lpo)]], bp[hb | tkb[k + (u << lpo)]]);
+          for (int u = 0; u < 8; ++u) mul_add(part[u], a[ha | tka[k + (u << lpo)]], bp[hb | tkb[k + (u << lpo)]]);
         }
-      } else {
-        for (int k = k0; k < (1 << kt); k += 1 << lpo) mul_add(acc[0], a[ha | tka[k]], bp[hb | tkb[k]]);
       }
+#pragma unroll
+      for (int h = 4; h > 0; h >>= 1)
+#pragma unroll
+        for (int u = 0; u < h; ++u) {
+          part[u].x += part[u + h].x;
+          part[u].y += part[u + h].y;
+        }
+      acc = part[0];
+    } else {  // few terms per lane: nK <= 8, so the tables hold every offset
+      for (int k = k0; k < (1 << kt); k += 1 << lpo) mul_add(acc, a[oa | tka[k]], bp[ob | tkb[k]]);
     }
-#pragma unroll
-    for (int h = 4; h > 0; h >>= 1)
-#pragma unroll
-      for (int u = 0; u < h; ++u) {
-        acc[u].x += acc[u + h].x;
-        acc[u].y += acc[u + h].y;
+    if (ENV)
+      for (int h = (1 << lpo) >> 1; h > 0; h >>= 1) {
+        acc.x += __shfl_xor(acc.x, h, 64);
+        acc.y += __shfl_xor(acc.y, h, 64);
       }
-    for (int h = (1 << lpo) >> 1; h > 0; h >>= 1) {
-      acc[0].x += __shfl_xor(acc[0].x, h, 64);
-      acc[0].y += __shfl_xor(acc[0].y, h, 64);
-    }
-    if ((i & ((1 << lpo) - 1)) == 0) c[o] = acc[0];
+    if ((i & ((1 << lpo) - 1)) == 0) c[o] = acc;
   }
 }
 
@@ -1343,19 +1356,20 @@ extern "C" int tedq_tn_contract(const void* a, int64_t a_bstride, const void* b,
 // elements, elements valid per batch row); records / records_dev: n_records
 // records of 8 int64, host and device copies; descs / descs_dev: the descriptor
 // table (n_descs rows), host and device copies.  Each step must have rank <= 12
-// operands and results, at most 2^max_k summed terms, and fit its arenas (all
-// checked on the host).  c_base >= 0: every result goes to that arena.
+// operands and results, at most 2^6 (ENV: 2^12) summed terms, and fit its arenas
+// (all checked on the host).  Without ENV every result goes to arena kSmallResults.
+template <bool ENV>
 static int launch_small(const char* what, const void* const* bases, const int64_t* strides, const int64_t* lens,
-                        int n_bases, const int64_t* records, const int64_t* records_dev, int n_records, int64_t batch,
-                        const int32_t* descs, const int32_t* descs_dev, int n_descs, int c_base, int max_k,
-                        void* stream) {
+                        const int64_t* records, const int64_t* records_dev, int n_records, int64_t batch,
+                        const int32_t* descs, const int32_t* descs_dev, int n_descs, void* stream) {
   if (bases == nullptr || strides == nullptr || lens == nullptr || records == nullptr || records_dev == nullptr ||
       descs == nullptr || descs_dev == nullptr || n_records < 0 || n_descs <= 0 || batch <= 0 || batch > 65535) {
     set_error("%s: bad arguments", what);
     return kBadArgument;
   }
   if (n_records == 0) return kOk;
-  TNBases tb = {};
+  TNBases<ENV> tb;
+  constexpr int n_bases = TNBases<ENV>::kCount;
   for (int i = 0; i < n_bases; ++i) {
     if (bases[i] == nullptr || strides[i] < 0 || lens[i] < 0) {
       set_error("%s: bad arena %d", what, i);
@@ -1373,7 +1387,8 @@ static int launch_small(const char* what, const void* const* bases, const int64_
     }
     const int nH = d.nb[0], nM = d.nb[1], nN = d.nb[2], nK = d.nb[3];
     const int64_t sa = 1ll << (nH + nM + nK), sb = 1ll << (nH + nN + nK), sc = 1ll << (nH + nM + nN);
-    const int64_t ic = c_base >= 0 ? c_base : rec[7];
+    const int64_t ic = ENV ? rec[7] : kSmallResults;
+    const int max_k = ENV ? 12 : kSmallSumBits;
     const bool shapes = nH + nM + nK <= 12 && nH + nN + nK <= 12 && nH + nM + nN <= 12 && nK <= max_k && rec[6] == sc;
     const bool in_a = rec[1] >= 0 && rec[1] < n_bases && rec[2] >= 0 && rec[2] + sa <= lens[rec[1]];
     const bool in_b = rec[3] >= 0 && rec[3] < n_bases && rec[4] >= 0 && rec[4] + sb <= lens[rec[3]];
@@ -1383,8 +1398,8 @@ static int launch_small(const char* what, const void* const* bases, const int64_
       return kBadArgument;
     }
   }
-  hipLaunchKernelGGL(k_tn_small_multi, dim3((unsigned)n_records, (unsigned)batch), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), tb, records_dev, descs_dev, c_base);
+  hipLaunchKernelGGL(k_tn_small_multi<ENV>, dim3((unsigned)n_records, (unsigned)batch), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), tb, records_dev, descs_dev);
   return check_launch(what);
 }
 
@@ -1393,8 +1408,8 @@ extern "C" int tedq_tn_contract_small_batch(const void* const* bases, const int6
                                             const int64_t* records, const int64_t* records_dev, int n_records,
                                             int64_t batch, const int32_t* descs, const int32_t* descs_dev,
                                             int n_descs, void* stream) {
-  return launch_small("tedq_tn_contract_small_batch", bases, strides, lens, 3, records, records_dev, n_records, batch,
-                      descs, descs_dev, n_descs, 2, 6, stream);
+  return launch_small<false>("tedq_tn_contract_small_batch", bases, strides, lens, records, records_dev, n_records,
+                             batch, descs, descs_dev, n_descs, stream);
 }
 
 // Five arenas, each record's last word naming its result's.
@@ -1402,8 +1417,8 @@ extern "C" int tedq_tn_small_environments(const void* const* bases, const int64_
                                           const int64_t* records, const int64_t* records_dev, int n_records,
                                           int64_t batch, const int32_t* descs, const int32_t* descs_dev, int n_descs,
                                           void* stream) {
-  return launch_small("tedq_tn_small_environments", bases, strides, lens, kSmallBases, records, records_dev, n_records,
-                      batch, descs, descs_dev, n_descs, -1, 12, stream);
+  return launch_small<true>("tedq_tn_small_environments", bases, strides, lens, records, records_dev, n_records, batch,
+                            descs, descs_dev, n_descs, stream);
 }
 
 // Eligibility of a forward step for tedq_tn_gate_backward (the k_tn_gate shape

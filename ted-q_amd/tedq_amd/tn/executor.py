@@ -698,7 +698,8 @@ class TNExecutor:
             if i == len(entries) or entries[i][0] != entries[start][0]:
                 bounds.append((start, i))
                 start = i
-        plan = {"recs": recs, "bounds": bounds, "offs": offs, "len": max(arena, 1), "dev": {}}
+        plan = {"recs": recs, "bounds": bounds, "offs": offs, "len": max(arena, 1), "dev": {},
+                "large": [(s, st) for s, st in enumerate(net.steps) if st.c not in offs]}
         self._small[key] = plan
         return plan
 
@@ -965,9 +966,7 @@ class TNExecutor:
         coef = self._run_coefs(plan, small, arena, leaves, buf, B, dev) if plan is not None else None
         if keep is not None:
             kept["arena"], kept["coef"] = arena, coef
-        for s, st in enumerate(net.steps):
-            if small is not None and st.c in small["offs"]:
-                continue
+        for s, st in small["large"] if small is not None else enumerate(net.steps):
             if plan is not None and s in plan["covered"]:
                 run = plan["first"].get(s)
                 if run is not None:
