@@ -731,16 +731,18 @@ class SVExecutor:
             coef = cols[m].contiguous()
             hip.call("tedq_sv_lambda_factored", hip.ptr(psi), hip.ptr(lam), B, self.n, 0, None, None,
                      self.zmasks[m], hip.ptr(coef), st)
+        if len(cols) == len(self.specs):
+            return lam
         # one-factor observables, when all of them have a gradient: one launch
-        up = {id(spec): g for spec, g in zip(self.specs, grads)}
+        done = ()
         one, recs, drecs = self._factored_records(dev).get(1, ((), None, None))
-        if one and all(up[id(spec)] is not None for spec in one):
-            coef = torch.stack([up[id(spec)].to(torch.float64).reshape(B) for spec in one], 1).contiguous()
-            hip.call("tedq_sv_lambda_factored_batch", hip.ptr(psi), hip.ptr(lam), B, self.n, _hptr(recs),
-                     hip.ptr(drecs), len(one), hip.ptr(coef), st)
-        else:
-            one = ()
-        done = {id(spec) for spec in one}
+        if one:
+            up = {id(spec): g for spec, g in zip(self.specs, grads)}
+            if all(up[id(spec)] is not None for spec in one):
+                coef = torch.stack([up[id(spec)].to(torch.float64).reshape(B) for spec in one], 1).contiguous()
+                hip.call("tedq_sv_lambda_factored_batch", hip.ptr(psi), hip.ptr(lam), B, self.n, _hptr(recs),
+                         hip.ptr(drecs), len(one), hip.ptr(coef), st)
+                done = {id(spec) for spec in one}
         for spec, g in zip(self.specs, grads):
             if g is None or spec.kind == "zexp" or id(spec) in done:
                 continue
