@@ -216,10 +216,10 @@ __global__ void __launch_bounds__(256) k_tn_run_balance(TNRunBases bases, const 
 }
 
 // One forward pass: workgroup (g, b) owns tile g of batch element b.
-// 256 threads and 32 KB of LDS at 2^12 elements: five workgroups per CU, whose
-// loads, matrices and stores overlap.  Measured on 2^25 elements with 8
-// matrices per pass: 189 us a pass (94 us + 15 us per
-// matrix), against 8 x 92 us step by step.
+// 256 threads, 32 KB of LDS at 2^12 elements and 8 B per matrix entry: four
+// workgroups per CU, whose loads, matrices and stores overlap.  Measured on
+// 2^25 elements: 128 us a pass with one matrix (a copy takes 102), 188 with 8,
+// 304 with 16, 534 with 32, against 92 us per matrix step by step.
 template <bool A3>
 __global__ void __launch_bounds__(256) k_tn_run_pass(const float2* __restrict__ X, int64_t x_bs,
                                                      float2* __restrict__ C, int64_t c_bs,
@@ -412,8 +412,8 @@ __device__ __forceinline__ void undo_op(float2* xt, float2* et, const float2* m,
 // partial sums written are per workgroup, not per tile.  EX may be EC when the
 // pass keeps the layout: a tile is read whole before it is written.
 // 512 threads, two tiles of 32 KB: two workgroups, 16 waves per CU.  Measured
-// on 2^25 elements with 8 matrices per pass: 503 us (130 us + 52 us per matrix),
-// against 8 x 152 us.
+// on 2^25 elements, with k_tn_run_env: 212 us a pass with one matrix, 572 with
+// 8, 1019 with 16, 1888 with 32, against 152 us per matrix step by step.
 template <bool A3>
 __global__ void __launch_bounds__(kBwdThreads) k_tn_run_bwd(const float2* __restrict__ C, int64_t c_bs,
                                                             const float2* EC, int64_t ec_bs, float2* EX,

@@ -417,8 +417,7 @@ def pass_kernel_source(name, words, adjoint, seed_masks=None, fresh=0, persisten
 
 # The table rows were written by another kernel: the first scalar load of each line misses this XCD's L2, one
 # stage after another.  The lines a pass reads are touched while its tile loads (persistent kernels: the next
-# tile's, of another circuit).  256 rows of a 20-qubit
-# training step: 38.5 -> 36.8 ms.
+# tile's, of another circuit).  256 rows of a 20-qubit training step: 38.5 -> 36.8 ms.
 _TOUCH, _TOUCH_NEXT, _TOUCHED = "  // touch table lines", "  // touch next table lines", "  // table lines touched"
 
 

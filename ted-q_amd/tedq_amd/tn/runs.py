@@ -22,8 +22,9 @@ import numpy as np
 
 MIN_WIRES = 9      # smallest large operand: a wave of 64 rows of an 8 x 8 op
 TILE_WIRES = 12    # largest tile: 2^12 amplitudes, 32 KB of LDS
-LOW_WIRES = 3      # lowest address bits of every tile: 64-byte segments (four cost 51 passes against 44 on a
-                   # 5x5 lattice and 37.6 against 37.0 ms: the longer segments do not repay the passes)
+LOW_WIRES = 3      # lowest address bits of every tile: 64-byte segments (four cost 51 forward passes against 44 on
+                   # a 5x5 lattice, 50 against 43 with gradients, and 37.6 against 37.0 ms: the longer segments do
+                   # not repay the passes)
 MAX_ARITY = 3
 MAX_FACTORS = 4
 MAX_INTERNAL = 3
