@@ -291,7 +291,9 @@ int tedq_tn_gate_backward(const void* ec, int64_t ec_bstride, const void* x, int
  * matrix entries, [4..16) input address bit of every slot, [16..28) slot and
  * [28..40) address bit of the tile's result bits, [40..60) and [72..92) input
  * and result address bits of the outer bits}.  tedq_tn_run_coefs forms the
- * matrices, tedq_tn_run_pass applies a pass (x and c distinct), and
+ * matrices (with coef_bstride of n_ops beyond the last matrix's end it also
+ * balances the scale that rounding products of several factors has, with that
+ * space as scratch), tedq_tn_run_pass applies a pass (x and c distinct), and
  * tedq_tn_run_backward undoes it from its result c (unitary matrices):
  * environment ec of the result -> ex of the input (ex may be ec when the
  * layout does not change), gate environments into env0 / env1. */
