@@ -768,7 +768,7 @@ class SVExecutor:
                 hip.call("tedq_sv_lambda_probs", hip.ptr(psi), hip.ptr(lam), B, self.n, k, _hptr(bits),
                          hip.ptr(gg), st)
             elif spec.kind == "state":
-                gs = g.to(torch.complex64).reshape(B, 2 ** self.n).contiguous()
+                gs = g.to(torch.complex64).reshape(B, 2 ** self.n).resolve_conj().resolve_neg().contiguous()
                 hip.call("tedq_sv_axpy", hip.ptr(lam), hip.ptr(gs), B, self.n, 0.5, st)
         return lam
 

@@ -1247,7 +1247,8 @@ class TNExecutor:
             return g.to(torch.float32).reshape(B, 1).to(torch.complex64)
         if spec.kind == "probs":
             return g.to(torch.float32).reshape(B, 1 << len(net.output)).to(torch.complex64)
-        return g.to(torch.complex64).reshape(B, -1).conj().contiguous()
+        # (conj() only marks a tensor; the kernels read its memory)
+        return g.to(torch.complex64).reshape(B, -1).conj().resolve_conj().resolve_neg().contiguous()
 
     def run_backward(self, rows, run, grads, grad_dtype=torch.float32):
         """Gradient [B, P] of sum_m <grads_m, out_m> by the reverse contraction tree of every network."""
